@@ -909,6 +909,31 @@ def test_gemm_h16_nonfinite_scales(capi, M, N):
     assert rel_fro(got, ref) < FRO_TOL, rel_fro(got, ref)
 
 
+@pytest.mark.parametrize("M,N,K", [(515, 8195, 2048),     # K split in 2: scalar fp32 partial stores
+                                   (513, 8198, 2048),     # ... rows of 4-byte alignment
+                                   (129, 33001, 256),     # one double batch, scalar fp16 stores
+                                   (257, 32772, 768),     # a one-row second tile, 8-byte rows
+                                   (65, 49155, 512)])     # 128-row tiles, scalar fp16 stores
+def test_gemm_h16q_ragged_columns(capi, M, N, K):
+    # converted-activation tiles whose rows of y are not whole 16-byte chunks,
+    # with a non-finite row and a non-finite last column (split plans write
+    # their NaN into the partials): every finite output within one fp16
+    # rounding plus 2K rounded fp32 additions of the fp64 product
+    g = rng(4900 + M)
+    xq, xs, wq, ws = _rand_operands(g, M, N, K)
+    xs[M - 1, 3], ws[N - 1, K // 32 - 1], ws[7, 0] = 0x7F80, 0xFFC0, 0x7F80
+    assert capi.gemm_s4_workspace_bytes(M, N, K) >= 2 * M * K
+    y = run_gemm(capi, xq, xs, wq, ws)
+    assert np.isnan(y[M - 1]).all() and np.isnan(y[:, [7, N - 1]]).all()
+    rows, cols = np.arange(M - 1), np.array([c for c in _sample(g, N, 600) if c not in (7, N - 1)] + [N - 2, N - 3])
+    assert np.isfinite(np.delete(y[:M - 1], [7, N - 1], axis=1)).all()
+    rows = rows[_sample(g, len(rows), 24)]
+    got, ref = y[np.ix_(rows, cols)], oracle.gemm_f64(xq[rows], xs[rows], wq[cols], ws[cols])
+    A = _abs_product(xq[rows], xs[rows], wq[cols], ws[cols])
+    bound = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64) + 2 * K * 2.0 ** -24 * A + 2.0 ** -25
+    assert (np.abs(got - ref) <= bound).all(), (M, N, K, float((np.abs(got - ref) / bound).max()))
+
+
 # Shapes the planner sends to the fp16-MFMA streaming kernel (gemm_h16s:
 # 32 < M <= 64, 224-column workgroups filling 7/8 to all of 256 CUs, i.e.
 # 49953 <= N <= 57344, K % 1024 == 0, 16-byte aligned operands): two 32-row

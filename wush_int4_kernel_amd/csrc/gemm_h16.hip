@@ -229,103 +229,6 @@ void gemm_h16w8_kernel(const uint8_t* __restrict__ xq, const uint16_t* __restric
     }
 }
 
-// ------------------------------------------------ pre-converted activations
-// For wide weight matrices every 256-row activation tile above is converted
-// again by each of the N/256 column tiles.  The workspace route converts the
-// activations once (h16_prep_a_kernel, M x K x 2 bytes of workspace), in the
-// MFMA fragment layout that gemm_h16q_kernel (gemm_h16q.hip) DMAs into LDS.
-// Same fp16 operands as gemm_h16w8_kernel; the K order within a block of four
-// groups differs (below), so the fp32 sums agree to rounding, not bit for bit.
-//
-// a16 layout: [32-row block][stage][K16 slice][64 lanes][16 B] (one block
-// and stage: the two 1 KiB operand fragments of v_mfma_f32_32x32x16_f16).
-// Within each block of 4 groups, stage 2 * (q & 1) + d / 2 of the block takes
-// dword d of group q at K16 slice d & 1 in lane half q >> 1 -- every stage
-// holds 32 codes of two groups, so that a wavefront converting a weight
-// column reads 32 contiguous bytes per half-wavefront for 4 stages.
-// ea[slice][row] = the row's power-of-two shift over the K slice, as the
-// per-tile conversion computes it.  Workgroups past mpad / 32 compute every
-// weight column's shift per slice, eb[slice][column] (npad columns, 0 past
-// N), once, instead of every 256 x 256 tile re-reading its columns' scales.
-// Grid: (mpad / 32 + npad / 256, splits): a workgroup converts 32 rows, or
-// takes 256 columns, of one slice.
-__global__ __launch_bounds__(256) void h16_prep_a_kernel(const uint8_t* __restrict__ xq,
-                                                         const uint16_t* __restrict__ xs,
-                                                         uint8_t* __restrict__ a16, int* __restrict__ ea,
-                                                         const uint16_t* __restrict__ ws, int* __restrict__ eb,
-                                                         int M, int N, int K, int groups_per_split, int mpad) {
-    const int G = K >> 5;
-    const int rb = blockIdx.x;
-    const int slice = blockIdx.y;
-    const int sg0 = slice * groups_per_split, sg1 = min(G, sg0 + groups_per_split);
-    const int tid = threadIdx.x;
-    if (rb >= mpad / 32) {
-        // weight column shifts: thread t, column 256 * (rb - mpad / 32) + t
-        const int npad = (N + kH16Tile - 1) / kH16Tile * kH16Tile;
-        const int c = (rb - mpad / 32) * 256 + tid;
-        int e = 0;
-        if (c < N) {
-            uint32_t mx, mx2;
-            const uint16_t* ps = ws + (size_t)c * G + sg0;
-            h16_row_max<true>(ps, ps, sg1 - sg0, mx, mx2);
-            e = h16_shift(mx);
-        }
-        eb[(size_t)slice * npad + c] = e;
-        return;
-    }
-    __shared__ int se[32];
-    {
-        // largest |scale| of each of the block's 32 rows over the slice: 8
-        // threads per row, 8 scales per load (slices are whole multiples of 8
-        // groups; scales 16-byte aligned)
-        const int r = tid >> 3, part = tid & 7;
-        const int row = rb * 32 + r;
-        u16x2 m2 = {0, 0};
-        if (row < M) {
-            const uint4* ps = reinterpret_cast<const uint4*>(xs + (size_t)row * G + sg0);
-            const int n8 = (sg1 - sg0) >> 3;
-#pragma unroll 4
-            for (int i = part; i < n8; i += 8) {
-                const uint4 v = ps[i];
-                m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(abs_bits2(v.x), abs_bits2(v.y)));
-                m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(abs_bits2(v.z), abs_bits2(v.w)));
-            }
-        }
-        uint32_t mx = max((uint32_t)m2.x, (uint32_t)m2.y);
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, 1));
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, 2));
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, 4));
-        if (part == 0) {
-            const int e = h16_shift(mx);
-            se[r] = e;
-            ea[(size_t)slice * mpad + row] = e;   // rows past M: never stored
-        }
-    }
-    __syncthreads();
-    // thread: row tid % 32 of groups sg0 + tid / 32, + 8, ...
-    const int rr = tid & 31;
-    const int row = rb * 32 + rr;
-    const int e = se[rr];
-#pragma unroll 4
-    for (int g = sg0 + (tid >> 5); g < sg1; g += 8) {
-        uint4 w = {0, 0, 0, 0};
-        float f = 0.0f;
-        if (row < M) {
-            w = *reinterpret_cast<const uint4*>(xq + (size_t)row * (K >> 1) + g * 16);
-            f = __uint_as_float((uint32_t)xs[(size_t)row * G + g] << 16);
-        }
-        const h2 sc = h16_scale(f, e);
-        const int q = g & 3;
-        const int st = (g & ~3) + 2 * (q & 1);                // stage of dwords 0, 1 (2, 3: st + 1)
-        uint8_t* dst = a16 + ((size_t)rb * G + st) * 2048;
-        const int L = rr + 32 * (q >> 1);
-        frag_write(dst, L, h16_codes(w.x, sc));
-        frag_write(dst + 1024, L, h16_codes(w.y, sc));
-        frag_write(dst + 2048, L, h16_codes(w.z, sc));
-        frag_write(dst + 3072, L, h16_codes(w.w, sc));
-    }
-}
-
 }  // namespace
 
 size_t gemm_h16_smem_bytes() { return 2 * kH16Buf + 2 * kH16Tile * sizeof(int); }
@@ -339,34 +242,6 @@ int gemm_h16_init_device() {
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_h16w8_kernel<false>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     return (int)e;
-}
-
-size_t gemm_h16a_workspace_bytes(int64_t M, int64_t N, int64_t K, int splits) {
-    const int64_t mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile;
-    const int64_t npad = (N + kH16Tile - 1) / kH16Tile * kH16Tile;
-    return (size_t)mpad * (size_t)K * 2 + (size_t)splits * (size_t)(mpad + npad) * sizeof(int);
-}
-
-int launch_gemm_h16a(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
-                     uint16_t* y, float* partial, int M, int N, int K, int splits, int groups_per_split,
-                     void* a_ws, bool rows128, hipStream_t stream) {
-    const int G = K >> 5;
-    if (M <= 0 || N <= 0 || K <= 0 || K % 256 != 0 || splits < 1 || groups_per_split <= 0 ||
-        groups_per_split % 8 != 0 || (long long)splits * groups_per_split < G ||
-        (long long)(splits - 1) * groups_per_split >= G || (splits > 1 && partial == nullptr) || a_ws == nullptr ||
-        ((reinterpret_cast<uintptr_t>(xs) | reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(a_ws)) &
-         15u) != 0)
-        return (int)hipErrorInvalidValue;
-    const int mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile;
-    const int npad = (N + kH16Tile - 1) / kH16Tile * kH16Tile;
-    uint8_t* a16 = static_cast<uint8_t*>(a_ws);
-    int* ea = reinterpret_cast<int*>(a16 + (size_t)mpad * K * 2);
-    int* eb = ea + (size_t)splits * mpad;
-    h16_prep_a_kernel<<<dim3((unsigned)(mpad / 32 + npad / 256), (unsigned)splits), 256, 0, stream>>>(
-        xq, xs, a16, ea, ws, eb, M, N, K, groups_per_split, mpad);
-    const int e = (int)hipGetLastError();
-    if (e != 0) return e;
-    return launch_gemm_h16q(a16, ea, eb, wq, ws, y, partial, M, N, K, groups_per_split, splits, rows128, stream);
 }
 
 int launch_gemm_h16(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,

@@ -1,45 +1,59 @@
-// gemm_h16q.hip -- the pre-converted-activation fp16-MFMA prefill GEMM with
-// one wavefront per SIMD (csrc/gemm_s4.cu:85-379 is the reference contract;
-// operands and numerics as in gemm_h16.hip).
+// gemm_h16q.hip -- the fp16-MFMA prefill GEMM with activations converted once
+// into a workspace and weights converted in registers, one wavefront per SIMD
+// (csrc/gemm_s4.cu:85-379 is the reference contract; operands and numerics as
+// in gemm_h16.hip).
 //
-// Workgroup: 4 wavefronts side by side, a 256 x 256 output tile, wavefront w
-// owning all 256 rows and weight columns 64w .. 64w + 63 (8 x 2 accumulator
-// blocks, 256 fp32 accumulators in AGPRs).  Because no other wavefront needs
-// its columns, a wavefront converts its weight codes straight into MFMA
-// B-operand registers: no LDS traffic for converted weights, no transpose.
-// The activations, converted once beforehand in the matching layout
-// (h16_prep_a_kernel<true>), are DMA'd into a 4-slot LDS ring four stages
-// ahead and read by all four wavefronts.
+// Workgroup: 4 wavefronts side by side over 256 weight columns, wavefront w
+// owning all of the tile's rows (256 or 128) and columns 64w .. 64w + 63.
+// Because no other wavefront needs its columns, a wavefront converts its
+// weight codes straight into MFMA operand registers: no LDS traffic for
+// converted weights.  The activations, converted once by h16_prep_kernel in
+// the matching layout, are DMA'd into a 4-slot LDS ring and read by all four.
+//
+// What bounds it on MI355X: power.  At L70 M=4096 an MFMA-only loop of the
+// same tile runs at 1.5-1.6 PFLOP/s with the clock near 1.5 GHz, so the MFMA
+// form matters: v_mfma_f32_16x16x32_f16 moves a third less accumulator data
+// per flop than the 32x32x16 form and the same loop ran 7-10% faster with it
+// (4096 x 16384 x 8192, operands in LDS: 907 -> 806 us).  The accumulators
+// are written in place by an asm MFMA: left to the compiler, tiles that do
+// not fill the AGPRs rotate them (each MFMA writing the next one's input),
+// which ran 40% slower.
 //
 // With one wavefront per SIMD there is no second wavefront to run the memory
-// work beside the MFMAs, so every wavefront runs a software pipeline of its
-// own, issued between its 32 MFMAs of stage t: stage t+1's activation
-// fragments, the conversion of stage t+1's weights, the DMAs of stage t+4.
-// One barrier per stage.  A wavefront's weight codes come in batches of four
-// stages, DMA'd into LDS two batches ahead and read into registers once per
-// batch (6 LDS reads per 4 stages, not 4 per stage: 4% faster at L70).  The
-// codes are DMA'd two batches at a time, each column's whole 128-byte line
-// per 8 lanes: with 32 bytes of 32 columns per DMA the kernel took 2-4%
-// longer (a load touching 32 lines costs the vector memory path about as much
-// as one reading them whole).
+// work beside the MFMAs, so each stage (one group of K per lane quarter, 32
+// in all) interleaves by hand: after each MFMA of stage t at most one LDS read
+// of stage t+1's activations, one or two VALU of the conversion of stage
+// t+1's weights, or one DMA of stage t+4 (DMAs issued four in a row held the
+// MFMAs up: 926 -> 870 us in the loop above when spread).  One barrier per stage.
 //
-// Every global load of the kernel is an LDS DMA issued by an asm statement
-// (activations, weight codes and scales, shifts), and the kernel orders them
-// itself: at the end of stage t a wavefront waits until its DMAs of stage
-// t+2 (and so everything it issued before them) have landed, then the barrier
-// publishes them.  Left to the compiler, LDS DMA is tracked per LDS object in
-// a small table; once the table overflows, every LDS read waits for all DMAs
-// in flight, and register loads mixed with such DMAs get waits counted
-// without them.
+// Stage layout: a weight column's 16 code bytes of group 4b + q sit in lane
+// quarter q, and stage 4b + s takes dword s of all four: a lane reads 16
+// contiguous bytes once per four stages and converts one scale for them.
 //
-// Outputs: fp16 through LDS (the ring is free after the last stage), so that
-// the global stores are 16-byte row chunks instead of one 2-byte store per
-// accumulator.
+// Weight codes come in double batches of 8 groups, each column's whole
+// 128-byte line per 8 lanes (a load touching 32 lines costs the vector memory
+// path about as much as one reading them whole), one DMA per stage.  Every
+// global load of the loop is an LDS DMA issued by asm that the compiler does
+// not see; the kernel counts them itself.  Every stage issues NA activation
+// DMAs and one code DMA, and stage 4 of each 8 one scale DMA more; at a
+// stage's end all but those of the last two stages have landed, so what a
+// stage issues is read three stages later at the earliest.
 //
-// Stage layout (h16_prep_a_kernel<true>): in each block of 4 groups a lane of
-// half h reads the 32 contiguous code bytes [32h, 32h + 32) of its column
-// (groups 2h and 2h + 1); stage s of the block takes dwords 2s and 2s + 1 of
-// them (K16 slices 0 and 1).
+// Outputs: fp16 through LDS (the ring and code buffers are free after the
+// last stage) as 8-byte writes -- the weights are the MFMA's row operand, so
+// a lane holds 4 consecutive columns of one row -- and 16-byte row chunks to
+// memory.  The shifts come from LDS and non-finite rows from NaN operands, so
+// an output costs four VALU (accumulator read, add, ldexp, half a conversion);
+// with per-output tests and 2-byte writes a 256 x 256 tile spent 15-20 us
+// outside its K loop, now about 10.
+//
+// Measured (layer with the fused transform, same box, against the 32x32x16
+// form with burst DMAs): K=8192 N=57344 M=4096 3179 -> 2679 us (1.45 PFLOP/s;
+// a library fp16 GEMM of the shape 2560-2850), M=256 238 -> 197, M=128 146 ->
+// 126; K=N=8192 M=4096 511 -> 431, M=512 116 -> 94; K=4096 N=24576 M=1024
+// 232 -> 185.
+#include <utility>
+
 #include "gemm_h16_device.h"
 #include "gemm_h16.h"
 #include "setup.h"
@@ -47,347 +61,444 @@
 namespace wush {
 namespace {
 
-#ifndef WUSH_H16Q_SCHED
-#define WUSH_H16Q_SCHED 1                        // explicit MFMA / LDS / VALU interleave
-#endif
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 
-// Tile id -> (row tile, column tile): workgroup i runs on XCD i % 8.  Each
-// XCD walks its column tiles in groups of 8, all row tiles of a group before
-// the next, so the workgroups in flight on an XCD share 8 weight column
-// tiles and a few activation row tiles in its L2.
-__device__ __forceinline__ void h16q_tile(uint32_t id, uint32_t NC, uint32_t NR, int& tm, int& tn) {
-    if ((NC & 7) != 0) {
-        tm = (int)(id / NC);
-        tn = (int)(id % NC);
-        return;
-    }
-    constexpr uint32_t kGroup = 8;
-    const uint32_t q = id >> 3, x = id & 7;
-    const uint32_t gsize = kGroup * NR;
-    const uint32_t g = q / gsize, w = q % gsize;
-    const uint32_t width = min(kGroup, (NC >> 3) - g * kGroup);
-    tm = (int)(w / width);
-    tn = (int)((g * kGroup + w % width) * 8 + x);
+// f(0), f(1), ..., f(N - 1) with compile-time arguments
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// RB: 32-row blocks per wavefront, 8 (256-row tiles) or 4 (128-row tiles, for
-// 64 < M <= 128: half the accumulators, the same weight conversion per stage).
+// c += a * b, accumulator in place.  The compiler does not know this is an
+// MFMA: the callers keep two instructions between a VALU write of an operand
+// and its use, and wait before reading c.
+__device__ __forceinline__ void mfma16_inplace(v4f& c, const h8& a, const h8& b) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+constexpr int kH16qStage = kH16Tile * 64;        // workspace bytes of one stage of a 256-row tile
+constexpr int kH16qGroupRows = 8;                // row tiles walked together (tile order)
+
+// Tile index s in walking order -> (row tile, column tile): groups of
+// kH16qGroupRows row tiles, all column tiles of a group before the next.
+// Workgroup i runs on XCD i % 8; each XCD takes a contiguous run of the
+// order, so the 32 workgroups in flight on it share 8 row tiles and a few
+// column tiles in its L2, for any tile counts.
+__device__ __forceinline__ void h16q_tile(int id, int NR, int NC, int& tm, int& tn) {
+    const int total = NR * NC;
+    const int q = total >> 3, r = total & 7, x = id & 7;
+    const int s = x * q + min(x, r) + (id >> 3);
+    const int g = s / (kH16qGroupRows * NC);
+    const int h = min(kH16qGroupRows, NR - g * kH16qGroupRows);
+    const int w = s - g * (kH16qGroupRows * NC);
+    tm = g * kH16qGroupRows + w % h;
+    tn = w / h;
+}
+
+// RB: 16-row blocks per wavefront, 16 (256-row tiles) or 8 (128-row tiles:
+// half the accumulators, the same weight conversion per stage).
 template <int RB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ ea, const int* __restrict__ eb,
                       const uint8_t* __restrict__ wq, const uint16_t* __restrict__ ws, uint16_t* __restrict__ y,
-                      float* __restrict__ partial, int M, int N, int K, int groups_per_split, int splits) {
-    // activation ring (4 stages) and, per wavefront, two double batches of
-    // weight codes [64 columns][128 B, pieces swizzled] and two batches of
-    // scales [2 columns][64 lanes][4 B]
-    __shared__ __align__(16) uint8_t sA[4][kH16Op];
-    __shared__ __align__(16) uint8_t sBc[2][4][8192];
-    __shared__ __align__(16) uint32_t sBs[2][4][128];
-    __shared__ __align__(16) int sh_e[512];      // [0, 256) rows, [256, 512) columns
+                      float* __restrict__ partial, int M, int N, int K, int groups_per_split) {
+    constexpr int TR = 16 * RB, TC = kH16Tile;
+    constexpr int NA = TR / 64;                  // activation DMAs per wavefront and stage
+    constexpr int NM = 4 * RB;                   // MFMAs per stage
+    constexpr int kSlot = TR * 64;               // LDS: activation ring of 4 slots,
+    constexpr int kCodes = 4 * kSlot;            // two double batches of codes per wavefront
+    constexpr int kScales = kCodes + 2 * 4 * 8192;   // [64 columns][128 B, pieces swizzled], their
+    constexpr int kShifts = kScales + 2 * 4 * 1024;  // scales [64 columns][8 groups], row and column shifts
+    __shared__ __align__(16) uint8_t smem[kShifts + 2048];
+    static_assert(4 * TR * 128 <= kScales, "outputs staged over the ring and code buffers");
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int half = lane >> 5;
-    const int l32 = lane & 31;
+    const int l16 = lane & 15, kq = lane >> 4;   // row or column of an operand, lane quarter
     const int GR = K >> 5;
     const int K2 = K >> 1;
-    const int limn = N - 1;
-    constexpr int TR = 32 * RB;                  // rows per tile
-    constexpr int NA = RB / 4;                   // activation row blocks DMA'd per wavefront
-    constexpr int kSlice = RB * 1024;            // bytes of one K16 slice of a stage's activations
-    const int NC = (N + kH16Tile - 1) / kH16Tile;
-    const int NR = (M + TR - 1) / TR;
+    const int NR = (M + TR - 1) / TR, NC = (N + TC - 1) / TC;
     // shifts and converted activations are laid out over 256-row padding
     const int mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile, npad = NC * kH16Tile;
-    const int per_slice = NC * NR;
-
-    const int id = blockIdx.x;
-    const int slice = id / per_slice;
+    const int slice = blockIdx.x / (NR * NC);
     int tm, tn;
-    h16q_tile((uint32_t)(id - slice * per_slice), (uint32_t)NC, (uint32_t)NR, tm, tn);
+    h16q_tile((int)blockIdx.x - slice * (NR * NC), NR, NC, tm, tn);
     const int m0 = tm * TR;
-    const int n0 = tn * kH16Tile;
+    const int n0 = tn * TC;
     const int gb = slice * groups_per_split;
     const int G = min(GR - gb, groups_per_split);
+    const uint32_t lds0 = lds_addr(smem);
 
-    // activation DMA of this wavefront: row blocks NA w .. NA w + NA - 1, both K16 slices
-    const uint8_t* asrc = a16 + ((size_t)((m0 >> 5) + NA * wave) * GR + gb) * 2048 + lane * 16;
-    const size_t arb = (size_t)GR * 2048;
-    auto issue_a = [&](int st, int slot) {
-        const uint8_t* src = asrc + (size_t)min(st, G - 1) * 2048;   // past the slice: the last stage
-        const uint32_t dst = lds_addr(sA[slot]) + NA * wave * 1024;
-#pragma unroll
-        for (int b = 0; b < NA; ++b) {
-            dma16(src + b * arb, dst + b * 1024);
-            dma16(src + b * arb + 1024, dst + kSlice + b * 1024);
-        }
+    // activation DMA of this wavefront: KiB NA w .. NA w + NA - 1 of a stage
+    const uint8_t* asrc = a16 + ((size_t)(m0 >> 8) * GR + gb) * kH16qStage + (m0 & 255) * 64 + wave * (NA * 1024);
+    const uint32_t avoff = lane * 16;
+    auto issue_a = [&](int st, int slot, int d) {    // past the slice: the last stage
+        dma16_uniform(asrc + (size_t)min(st, G - 1) * kH16qStage + d * 1024, avoff,
+                      lds0 + slot * kSlot + wave * (NA * 1024) + d * 1024);
     };
-    // this lane's two weight columns (blocks 2w and 2w + 1): their scales
-    const int colA = min(n0 + wave * 64 + l32, limn);
-    const int colB = min(n0 + wave * 64 + 32 + l32, limn);
-    const uint16_t* sa = ws + (size_t)colA * GR + gb + 2 * half;
-    const uint16_t* sb = ws + (size_t)colB * GR + gb + 2 * half;
-    // Weight codes come in double batches (8 groups, each column's whole
-    // 128-byte line): DMA k of a double batch reads columns 8k .. 8k+7 of the
-    // wavefront's 64, 8 lanes a line.  Lane l fetches piece (l % 8) ^ f(c) of
-    // column c = 8k + l / 8, so that piece p of column c sits at
-    // 128 c + 16 (p ^ f(c)) with f(c) = (c / 2) % 8: 16 consecutive readers
-    // (columns c .. c+15, one piece) hit distinct banks.
-    const uint32_t cbase = (uint32_t)(n0 + wave * 64);
-    auto issue_db = [&](int d, int buf) {
-        const int o = min(d * 2 * kH16Batch, G - 2 * kH16Batch);
-        const uint8_t* base = wq + (size_t)(gb + o) * 16;
-        const uint32_t c0 = lds_addr(sBc[buf][wave]);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int c = 8 * k + (lane >> 3);
-            const int p = (lane & 7) ^ ((c >> 1) & 7);
-            const uint32_t col = min(cbase + (uint32_t)c, (uint32_t)limn);
-            dma16(base + (size_t)col * K2 + p * 16, c0 + 1024 * k);
-        }
+    // Code DMA k of a double batch: columns 8k .. 8k+7 of the wavefront's 64.
+    // Lane l fetches piece (l % 8) ^ f(c) of column c = 8k + l / 8, so that
+    // piece p of column c sits at 128 c + 16 (p ^ f(c)) with f(c) = (c / 2) %
+    // 8: 16 consecutive readers (columns c .. c+15, one piece) hit distinct
+    // banks.  Columns past N read column N - 1.
+    const int col0 = n0 + wave * 64;
+    auto issue_c = [&](int d, int buf, int k) {
+        const int o = min(d * 8, G - 8);
+        const int c = 8 * k + (lane >> 3);
+        const int p = (lane & 7) ^ ((c >> 1) & 7);
+        const int col = min(col0 + c, N - 1);
+        dma16(wq + (size_t)col * K2 + (size_t)(gb + o) * 16 + p * 16,
+              lds0 + kCodes + (buf * 4 + wave) * 8192 + k * 1024);
     };
-    auto issue_s = [&](int b, int buf) {
-        const int o = min(b * kH16Batch, G - kH16Batch);
-        const uint32_t s = lds_addr(sBs[buf][wave]);
-        dma4(sa + o, s);
-        dma4(sb + o, s + 256);
+    const uint16_t* ssrc = ws + (size_t)min(col0 + lane, N - 1) * GR + gb;
+    auto issue_s = [&](int d, int buf) {
+        dma16(ssrc + min(d * 8, G - 8), lds0 + kScales + (buf * 4 + wave) * 1024);
     };
-    v16f acc[RB][2];
-    h8 fa[2][2][RB];                             // [register set][K16 slice][row block]
-    h8 fb[2][2][2];                              // [register set][K16 slice][column block]
-    auto read_frag = [&](int slot, int P, int kk, int i) {
-        fa[P][kk][i] = frag_read(sA[slot] + kk * kSlice + i * 1024, lane);
+
+    v4f acc[RB][4];
+    h8 fa[2][RB];                                // [register set][row block]
+    uint32_t fb[2][4][4];                        // [register set][column block][dword]
+    const uint8_t* abase = smem + lane * 16;
+    auto read_a = [&](int P, int slot, int i) {
+        fa[P][i] = *reinterpret_cast<const h8*>(abase + slot * kSlot + i * 1024);
     };
-    int eA = 0, eB = 0;
-    // A weight batch in registers, read from its LDS buffer once: this
-    // lane's 32 code bytes of each of its two columns, and their scales
-    // (two bf16 per column: groups 2h and 2h + 1 of the batch's block).
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    // A weight batch (four stages) in registers: per column block the lane's
+    // 16 code bytes (group 4b + kq) and their fp16 scale
     struct Batch {
-        u32x4 c[2][2];                           // [column block][16-byte half]
-        uint32_t s[2];
+        u32v4 c[4];
+        h2 s[4];
     };
-    // batch b: double batch b / 2 in code buffer (b / 2) & 1, its half b & 1;
-    // scales in buffer b & 1
-    const int fsw = (l32 >> 1) & 7;                // f(c) of both the lane's columns
+    Batch R[2];
+    uint32_t sraw[4];
+    int ecol[4];
+    const int fsw = (l16 >> 1) & 7;              // f(c) of the lane's columns
     auto read_batch = [&](int b, Batch& r) {
-        const uint8_t* cb = sBc[(b >> 1) & 1][wave];
+        const uint8_t* cb = smem + kCodes + (((b >> 1) & 1) * 4 + wave) * 8192 + l16 * 128 +
+                            16 * ((4 * (b & 1) + kq) ^ fsw);
+        const uint8_t* sb = smem + kScales + (((b >> 1) & 1) * 4 + wave) * 1024 + l16 * 16 + 2 * (4 * (b & 1) + kq);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int c = (k >> 1) * 32 + l32;       // column block A, then B
-            const int p = 4 * (b & 1) + 2 * half + (k & 1);
-            r.c[k >> 1][k & 1] = *reinterpret_cast<const u32x4*>(cb + c * 128 + 16 * (p ^ fsw));
+        for (int j = 0; j < 4; ++j) {
+            r.c[j] = *reinterpret_cast<const u32v4*>(cb + j * 2048);
+            sraw[j] = *reinterpret_cast<const uint16_t*>(sb + j * 256);
         }
-        r.s[0] = sBs[b & 1][wave][lane];
-        r.s[1] = sBs[b & 1][wave][64 + lane];
     };
-    // stage s (0-3) of a batch, column block jb -> B operands of register set P
-    auto convert_b = [&](int P, const Batch& r, int s, int jb) {
-        const uint32_t sv = r.s[jb];
-        const float f = __uint_as_float((s & 2) ? (sv & 0xffff0000u) : (sv << 16));
-        const h2 sc = h16_scale(f, jb ? eB : eA);
-        const u32x4& c = r.c[jb][s >> 1];
-        fb[P][0][jb] = __builtin_bit_cast(h8, h16_codes((s & 1) ? c[2] : c[0], sc));
-        fb[P][1][jb] = __builtin_bit_cast(h8, h16_codes((s & 1) ? c[3] : c[1], sc));
+    auto make_scale = [&](Batch& r, int j) { r.s[j] = h16_scale(__uint_as_float(sraw[j] << 16), ecol[j]); };
+    // Step k (of 52) of h16_codes for stage s of batch r: column block k / 13
+    // into register set P, one VALU instruction a step.
+    uint32_t w8 = 0;
+    h2 pr[4];
+    auto convert_step = [&](int P, const Batch& r, int s, int k) {
+        const int jb = k / 13, q = k % 13;
+        const uint32_t w = r.c[jb][s];
+        const h2 b0 = {(_Float16)1032.0f, (_Float16)1032.0f};
+        const h2 b1 = {(_Float16)72.0f, (_Float16)72.0f};
+        if (q == 0) w8 = w >> 8;
+        else if (q == 1) pr[0] = __builtin_bit_cast(h2, h16_nib(w, 0x000F000Fu, 0x64086408u));
+        else if (q == 2) pr[1] = __builtin_bit_cast(h2, h16_nib(w, 0x00F000F0u, 0x54805480u));
+        else if (q == 3) pr[2] = __builtin_bit_cast(h2, h16_nib(w8, 0x000F000Fu, 0x64086408u));
+        else if (q == 4) pr[3] = __builtin_bit_cast(h2, h16_nib(w8, 0x00F000F0u, 0x54805480u));
+        else if (q < 9) pr[q - 5] = pr[q - 5] - ((q & 1) ? b0 : b1);
+        else fb[P][jb][q - 9] = __builtin_bit_cast(uint32_t, (h2)(pr[q - 9] * r.s[jb]));
     };
-    Batch R0, R1;                                // batches in LDS buffers 0 and 1
 
-    // Prologue: shifts, activation stages 0-3, weight batches 0 and 1.
-    if (64 * wave < TR)                          // the tile's rows, padded rows included
-        dma4(ea + (size_t)slice * mpad + m0 + wave * 64 + lane, lds_addr(sh_e + wave * 64));
-    dma4(eb + (size_t)slice * npad + n0 + wave * 64 + lane, lds_addr(sh_e + 256 + wave * 64));
-    issue_a(0, 0);
-    issue_a(1, 1);
-    issue_a(2, 2);
-    issue_a(3, 3);
-    issue_db(0, 0);
+    // Prologue: shifts, double batch 0, then "stages" -4 .. -1 of the loop's
+    // DMA pattern (activation stages 0-3, half of double batch 1).
+    if (64 * wave < TR)
+        dma4(ea + (size_t)slice * mpad + m0 + wave * 64 + lane, lds0 + kShifts + wave * 256);
+    dma4(eb + (size_t)slice * npad + n0 + wave * 64 + lane, lds0 + kShifts + 1024 + wave * 256);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) issue_c(0, 0, k);
     issue_s(0, 0);
     issue_s(1, 1);
-    WUSH_WAIT_VMCNT(2);                          // all but batch 1's scales
-    WUSH_LDS_BARRIER();
-    eA = sh_e[256 + wave * 64 + l32];
-    eB = sh_e[256 + wave * 64 + 32 + l32];
-    read_batch(0, R0);
-    convert_b(0, R0, 0, 0);
-    convert_b(0, R0, 0, 1);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int s = 0; s < 4; ++s) {
 #pragma unroll
-        for (int i = 0; i < RB; ++i) read_frag(0, 0, kk, i);
+        for (int d = 0; d < NA; ++d) issue_a(s, s, d);
+        issue_c(1, 1, s);
+    }
+    constexpr int kInFlight = 2 * (NA + 1);      // DMAs of two stages
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = (v16f){0.0f};
+        for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    WUSH_WAIT_VMCNT(kInFlight);
+    WUSH_LDS_BARRIER();
+    const int* sh_e = reinterpret_cast<const int*>(smem + kShifts);   // minus the shift; [256..] columns
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ecol[j] = -sh_e[256 + wave * 64 + j * 16 + l16];
+    read_batch(0, R[0]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) make_scale(R[0], j);
+    static_for<52>([&](auto k) { convert_step(0, R[0], 0, k.value); });
+#pragma unroll
+    for (int i = 0; i < RB; ++i) read_a(0, 0, i);
     __builtin_amdgcn_sched_barrier(0);
 
-    for (int s0 = 0; s0 < G; s0 += 2 * kH16Batch) {
-        // fully unrolled: the batch registers and register sets are picked by j
-#pragma clang loop unroll(full)
-        for (int j = 0; j < 2 * kH16Batch; ++j) {
+    for (int s0 = 0; s0 < G; s0 += 8) {
+        // fully unrolled: register sets, slots and batches are picked by j
+        static_for<8>([&](auto jc) {
+            constexpr int j = jc.value, P = j & 1;
             const int t = s0 + j;
-            const int P = j & 1;
-            issue_a(t + 4, j & 3);               // into the slot stage t left
-            // a batch buffer's next batch once its last stage is converted
-            // double batch s0 / 8 + 1 once batch s0 / 4 - 1 (its buffer's
-            // last) is in registers; batch scales as before
-            if (j == 3) {
-                issue_db(s0 / (2 * kH16Batch) + 1, (s0 / (2 * kH16Batch) + 1) & 1);
-                issue_s(s0 / kH16Batch + 2, 0);
-            }
-            if (j == 7) issue_s(s0 / kH16Batch + 3, 1);
-            // stage t + 1's weights: batch (t + 1) / 4, in LDS buffer
-            // ((t + 1) / 4) & 1, stage (j + 1) % 4 of it.  A batch goes into
-            // registers at the stage before its first, ahead of that stage's
-            // fragment reads (LDS returns in order: read late, the
-            // conversion would wait for all of them).
-            if (j == 3) read_batch(s0 / kH16Batch + 1, R1);
-            if (j == 7) read_batch(s0 / kH16Batch + 2, R0);
-            const Batch& Rc = (j < 3 || j == 7) ? R0 : R1;
-            const int sc = (j + 1) & 3;
-            // 32 MFMAs of stage t; between them stage t+1's 16 activation
-            // fragment reads (past the last stage they read a stale slot,
-            // unused) and its weight conversions
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-                for (int i = 0; i < RB; ++i) {
-#pragma unroll
-                    for (int jb = 0; jb < 2; ++jb) {
-                        acc[i][jb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[P][kk][i], fb[P][kk][jb],
-                                                                            acc[i][jb], 0, 0, 0);
-                        const int m = kk * 2 * RB + i * 2 + jb;   // MFMA index in the stage
-                        if (m < 2 * RB) read_frag((j + 1) & 3, P ^ 1, m / RB, m % RB);
-                        if (m == 2 * RB) convert_b(P ^ 1, Rc, sc, 0);
-                        if (m == 3 * RB) convert_b(P ^ 1, Rc, sc, 1);
-                    }
+            Batch& Rc = R[((j + 1) >> 2) & 1];   // batch of stage t + 1
+            Batch& Rn = R[((j + 2) >> 2) & 1];   // batch read at j = 2 and 6
+            static_for<NM>([&](auto mc) {
+                constexpr int m = mc.value, i = m >> 2, jb = m & 3;
+                mfma16_inplace(acc[i][jb],
+                               __builtin_bit_cast(h8, (u32v4){fb[P][jb][0], fb[P][jb][1], fb[P][jb][2], fb[P][jb][3]}),
+                               fa[P][i]);
+                // stage t + 4 into the slot of stage t, whose fragments were
+                // all read (and waited for) before the last barrier
+                if constexpr (m % (NM / 4) == 1 && m / (NM / 4) < NA) issue_a(t + 4, j & 3, m / (NM / 4));
+                // double batch d's buffer is free once its second batch is in
+                // registers (j = 2): the codes of d + 2 from j = 4 on
+                if constexpr (m == NM * 7 / 8) {
+                    if constexpr (j < 4) issue_c(s0 / 8 + 1, (s0 / 8 + 1) & 1, j + 4);
+                    else issue_c(s0 / 8 + 2, (s0 / 8) & 1, j - 4);
                 }
-            }
-#if WUSH_H16Q_SCHED
-            // a batch's reads, then per MFMA one activation fragment read over
-            // the first 16; the conversion VALU spread over all
-#pragma unroll
-            for (int m = 0; m < 4 * RB; ++m) {
-                if (m == 0 && (j == 3 || j == 7)) __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);   // DS read: batch
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-                if (m < 2 * RB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // DS read: activations
-                if (m < 2 * RB) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);   // VALU
-                else __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-            }
-#endif
-            // activation stage t + 2 landed: the DMAs issued after its 4 are
-            // stage t+3's and t+4's (8) plus the batches of stages t-2 .. t
-            // (issued after their stage's activations); at the first stages
-            // the count also covers the prologue's DMAs
-            // (10 weight DMAs at j = 3, 2 at j = 7)
-            const int nb = (j >= 3 && j <= 5) ? 10 : (j == 7 || j <= 1) ? 2 : 0;
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (NA == 2) {
-                if (nb == 0) WUSH_WAIT_VMCNT(8);
-                else if (nb == 2) WUSH_WAIT_VMCNT(10);
-                else WUSH_WAIT_VMCNT(18);
-            } else {
-                static_assert(NA == 1, "activation DMAs per stage: 2 * NA");
-                if (nb == 0) WUSH_WAIT_VMCNT(4);
-                else if (nb == 2) WUSH_WAIT_VMCNT(6);
-                else WUSH_WAIT_VMCNT(14);
-            }
+                if constexpr (j == 4 && m == NM / 2 + 2) issue_s(s0 / 8 + 2, (s0 / 8) & 1);
+                if constexpr ((j & 3) == 2) {
+                    if constexpr (m == 0) read_batch(s0 / 4 + (j >> 2) + 1, Rn);
+                    if constexpr (m >= NM / 2 && (m - NM / 2) % (NM / 8) == 0) make_scale(Rn, (m - NM / 2) / (NM / 8));
+                }
+                // the activation reads end NM / 8 MFMAs before the stage, so
+                // that the barrier's LDS wait finds them done (past the last
+                // stage they read a stale slot, unused)
+                constexpr int kReadMs = NM - NM / 8;
+                static_for<RB>([&](auto r) {
+                    if constexpr (r.value * kReadMs / RB == m) read_a(P ^ 1, (j + 1) & 3, r.value);
+                });
+                constexpr int k0 = (m * 52 + NM - 1) / NM, k1 = ((m + 1) * 52 + NM - 1) / NM;
+                static_for<k1 - k0>([&](auto k) { convert_step(P ^ 1, Rc, (j + 1) & 3, k0 + k.value); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (j == 4 || j == 5) WUSH_WAIT_VMCNT(kInFlight + 1);   // the scale DMA of j = 4
+            else WUSH_WAIT_VMCNT(kInFlight);
             WUSH_LDS_BARRIER();
             __builtin_amdgcn_sched_barrier(0);
-        }
+        });
     }
     // The stages past the slice DMA'd copies of its last stage into the ring
     WUSH_WAIT_VMCNT(0);
+    asm volatile("s_nop 15\n\ts_nop 15");        // the last MFMAs' results
     __syncthreads();                             // the ring is free
 
-    const int ecA = sh_e[256 + wave * 64 + l32];
-    const int ecB = sh_e[256 + wave * 64 + 32 + l32];
-    auto out_value = [&](int i, int jb, int q, int e_row) {
-        const int e_col = jb ? ecB : ecA;
-        float v = __builtin_ldexpf(acc[i][jb][q], -(e_row + e_col));
-        if (e_row == kH16NonFinite || e_col == kH16NonFinite) v = __builtin_nanf("");
+    const int wn0 = n0 + wave * 64;
+    int er[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) er[i] = sh_e[i * 16 + l16];
+    const int4* ec4 = reinterpret_cast<const int4*>(sh_e + 256 + wave * 64 + 4 * kq);
+    // accumulator [i][j][q]: row 16 i + l16, column 16 j + 4 kq + q
+    auto out4 = [&](int i, int j, const int4& ec) {
+        v4f v;
+        v[0] = __builtin_ldexpf(acc[i][j][0], er[i] + ec.x);
+        v[1] = __builtin_ldexpf(acc[i][j][1], er[i] + ec.y);
+        v[2] = __builtin_ldexpf(acc[i][j][2], er[i] + ec.z);
+        v[3] = __builtin_ldexpf(acc[i][j][3], er[i] + ec.w);
         return v;
     };
+    // columns with a non-finite scale (one per lane): NaN over what was stored
+    uint64_t bad = __ballot(sh_e[256 + wave * 64 + lane] == kH16NonFinite);
     if (partial != nullptr) {
-        // fp32 partials of a K slice: one store per accumulator
+        // fp32 partials of a K slice, 64 contiguous bytes per row and instruction
+        const bool vec = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(partial) & 15u) == 0;
+        float* prow = partial + ((size_t)slice * M + m0 + l16) * N + wn0 + 4 * kq;
 #pragma unroll
-        for (int jb = 0; jb < 2; ++jb) {
-            const int col = n0 + wave * 64 + jb * 32 + l32;
+        for (int j = 0; j < 4; ++j) {
+            const int4 ec = ec4[j * 4];
+            const int n = wn0 + j * 16 + 4 * kq;
 #pragma unroll
-            for (int i = 0; i < RB; ++i)
+            for (int i = 0; i < RB; ++i) {
+                const v4f v = out4(i, j, ec);
+                if (m0 + i * 16 + l16 < M) {
+                    float* dst = prow + (size_t)(i * 16) * N + j * 16;
+                    if (vec) {
+                        if (n < N) *reinterpret_cast<v4f*>(dst) = v;
+                    } else {
 #pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    const int rl = i * 32 + 8 * (q >> 2) + 4 * half + (q & 3);
-                    const int row = m0 + rl;
-                    const float v = out_value(i, jb, q, sh_e[rl]);
-                    if (row < M && col < N) partial[((size_t)slice * M + row) * N + col] = v;
+                        for (int e = 0; e < 4; ++e)
+                            if (n + e < N) dst[e] = v[e];
+                    }
                 }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (bad != 0) {
+            WUSH_WAIT_VMCNT(0);
+            for (; bad != 0; bad &= bad - 1) {
+                const int n = wn0 + __builtin_ctzll(bad);
+                for (int m = m0 + lane; m < min(M, m0 + TR); m += 64)
+                    if (n < N) partial[((size_t)slice * M + m) * N + n] = __builtin_nanf("");
+            }
         }
         return;
     }
-    // fp16: each wavefront's 256 x 64 outputs through its ring slot (16 KiB),
-    // 128 rows at a time: 2-byte LDS writes in the accumulator layout, then
-    // 16-byte reads and stores of 8 columns of a row
+    // fp16: each wavefront's TR x 64 outputs through LDS, 128 bytes a row,
+    // 16-byte chunk c of row r at chunk c ^ (r % 8)
+    uint8_t* stg = smem + wave * (TR * 128);
+    uint8_t* wst = stg + l16 * 128 + (kq & 1) * 8;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int4 ec = ec4[j * 4];
+        uint8_t* w = wst + ((j * 2 + (kq >> 1)) ^ (l16 & 7)) * 16;
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+            *reinterpret_cast<h4*>(w + i * 16 * 128) = __builtin_convertvector(out4(i, j, ec), h4);
+        __builtin_amdgcn_sched_barrier(0);       // one column block at a time
+    }
     const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-    uint8_t* stg = sA[wave];
-    uint8_t* wbase = stg + 4 * half * 128 + l32 * 2;                 // row 4 * half, column l32
-    const uint8_t* rbase = stg + (lane >> 3) * 128 + (lane & 7) * 16;
-    const int* erow = sh_e + 4 * half;
+    const int r0 = lane >> 3, cc = lane & 7;
+    const int n = wn0 + cc * 8;
+    const uint8_t* rst = stg + r0 * 128 + (cc ^ r0) * 16;    // row 8 k + r0: (8 k + r0) % 8 == r0
+    uint16_t* yrow = y + (size_t)(m0 + r0) * N + n;
 #pragma unroll
-    for (int pass = 0; pass < RB / 4; ++pass) {
+    for (int k = 0; k < TR / 8; ++k) {
+        const uint4 v = *reinterpret_cast<const uint4*>(rst + k * 1024);
+        if (m0 + 8 * k + r0 < M) {
+            uint16_t* dst = yrow + (size_t)(8 * k) * N;
+            if (vec) {
+                if (n < N) *reinterpret_cast<uint4*>(dst) = v;
+            } else {
+                const uint32_t d[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-            const int i = 4 * pass + i4;
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const int4 er4 = *reinterpret_cast<const int4*>(erow + 32 * i + 8 * q4);
-                const int e_r[4] = {er4.x, er4.y, er4.z, er4.w};
-#pragma unroll
-                for (int jb = 0; jb < 2; ++jb)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const uint16_t h = f32_to_f16_bits(out_value(i, jb, 4 * q4 + r, e_r[r]));
-                        *reinterpret_cast<uint16_t*>(wbase + (32 * i4 + 8 * q4 + r) * 128 + 64 * jb) = h;
-                    }
-            }
-            __builtin_amdgcn_sched_barrier(0);   // one row block at a time
-        }
-        const int row0 = m0 + 128 * pass + (lane >> 3);
-        const int col = n0 + wave * 64 + (lane & 7) * 8;
-        uint16_t* dst0 = y + (size_t)row0 * N + col;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const uint4 v = *reinterpret_cast<const uint4*>(rbase + k * 1024);
-            if (row0 + 8 * k < M) {
-                uint16_t* dst = dst0 + (size_t)(8 * k) * N;
-                if (vec && col + 8 <= N) {
-                    *reinterpret_cast<uint4*>(dst) = v;
-                } else {
-                    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (col + e < N) dst[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
-                }
+                for (int e = 0; e < 8; ++e)
+                    if (n + e < N) dst[e] = (uint16_t)(d[e >> 1] >> (16 * (e & 1)));
             }
         }
-        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (bad != 0) {
+        WUSH_WAIT_VMCNT(0);
+        for (; bad != 0; bad &= bad - 1) {
+            const int c = wn0 + __builtin_ctzll(bad);
+            for (int m = m0 + lane; m < min(M, m0 + TR); m += 64)
+                if (c < N) y[(size_t)m * N + c] = 0x7e00;
+        }
+    }
+}
+
+// ------------------------------------------------ pre-converted activations
+// a16 layout: [256-row tile][stage][16-row block][64 lanes][16 B]; stage
+// 4b + s, lane (row % 16) + 16 q holds the 8 fp16 operands of dword s of group
+// 4b + q.  ea[slice][row] and eb[slice][column] hold MINUS the power-of-two
+// shift over the K slice, or kH16NonFinite for a column with a non-finite
+// scale (its outputs are set to NaN); a row with one gets NaN operands.
+// Rows past M are zero (shift 0 for them and for columns past N).
+//
+// Workgroups [0, na) convert 32 rows by `chunk` groups of one slice each
+// (scanning the rows' scales of the slice first, 8 threads a row); the rest
+// take 32 weight columns' shifts of one slice.  A wavefront load reads 8 whole
+// 128-byte lines of codes and its stores write whole 128-byte lines.
+// HBM-bound: 4096 x 8192 in 17.4 us (4.9 TB/s over 84 MB), against 28.5 us
+// with each thread loading 16 bytes of its own row and one 32-row block per
+// workgroup (most of a wave of workgroups idle at small M).
+__device__ __forceinline__ uint32_t slice_scale_max(const uint16_t* p, int n, int part) {
+    u16x2 m2 = {0, 0};
+    const uint4* p4 = reinterpret_cast<const uint4*>(p);
+#pragma unroll 4
+    for (int i = part; i < (n >> 3); i += 8) {
+        const uint4 v = p4[i];
+        m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(abs_bits2(v.x), abs_bits2(v.y)));
+        m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(abs_bits2(v.z), abs_bits2(v.w)));
+    }
+    return max((uint32_t)m2.x, (uint32_t)m2.y);
+}
+
+constexpr int kPrepChunk = 32;                   // groups per converting workgroup
+
+__global__ __launch_bounds__(256) void h16_prep_kernel(const uint8_t* __restrict__ xq,
+                                                       const uint16_t* __restrict__ xs,
+                                                       uint8_t* __restrict__ a16, int* __restrict__ ea,
+                                                       const uint16_t* __restrict__ ws, int* __restrict__ eb,
+                                                       int M, int N, int G, int groups_per_split, int mblocks,
+                                                       int nblocks, int chunks, int na) {
+    const int tid = threadIdx.x;
+    const int r = tid >> 3, part = tid & 7;
+    const bool wside = (int)blockIdx.x >= na;
+    const int id = wside ? blockIdx.x - na : blockIdx.x;
+    const int blk = id % (wside ? nblocks : mblocks);
+    const int rest = id / (wside ? nblocks : mblocks);
+    const int chunk = wside ? 0 : rest % chunks;
+    const int slice = wside ? rest : rest / chunks;
+    const int sg0 = slice * groups_per_split, sg1 = min(G, sg0 + groups_per_split);
+    const int row = blk * 32 + r;
+    const bool ok = row < (wside ? N : M);
+    uint32_t mx = ok ? slice_scale_max((wside ? ws : xs) + (size_t)row * G + sg0, sg1 - sg0, part) : 0x3f80u;
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 1));
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 2));
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 4));
+    const int e = h16_shift(mx);
+    if (wside) {
+        if (part == 0) eb[(size_t)slice * (nblocks * 32) + row] = !ok ? 0 : e == kH16NonFinite ? kH16NonFinite : -e;
+        return;
+    }
+    if (part == 0 && chunk == 0) ea[(size_t)slice * (mblocks * 32) + row] = !ok || e == kH16NonFinite ? 0 : -e;
+    const uint8_t* q = xq + (size_t)row * G * 16;
+    const uint16_t* s = xs + (size_t)row * G;
+    uint8_t* dst = a16 + (size_t)(blk >> 3) * G * kH16qStage + (blk & 7) * 2048 + (r >> 4) * 1024 + (r & 15) * 16;
+    const int g1 = min(sg1, sg0 + (chunk + 1) * kPrepChunk);
+#pragma unroll 4
+    for (int g = sg0 + chunk * kPrepChunk + part; g < g1; g += 8) {
+        uint4 w = {0, 0, 0, 0};
+        float f = 0.0f;
+        if (ok) {
+            w = *reinterpret_cast<const uint4*>(q + (size_t)g * 16);
+            f = __uint_as_float((uint32_t)s[g] << 16);
+        }
+        if (e == kH16NonFinite) f = __builtin_nanf("");
+        const h2 sc = h16_scale(f, e);
+        uint8_t* d = dst + (size_t)(g & ~3) * kH16qStage + (g & 3) * 256;
+        *reinterpret_cast<uint4*>(d) = h16_codes(w.x, sc);
+        *reinterpret_cast<uint4*>(d + kH16qStage) = h16_codes(w.y, sc);
+        *reinterpret_cast<uint4*>(d + 2 * kH16qStage) = h16_codes(w.z, sc);
+        *reinterpret_cast<uint4*>(d + 3 * kH16qStage) = h16_codes(w.w, sc);
     }
 }
 
 }  // namespace
 
-int launch_gemm_h16q(const uint8_t* a16, const int* ea, const int* eb, const uint8_t* wq, const uint16_t* ws,
-                     uint16_t* y, float* partial, int M, int N, int K, int groups_per_split, int splits,
-                     bool rows128, hipStream_t stream) {
+size_t gemm_h16a_workspace_bytes(int64_t M, int64_t N, int64_t K, int splits) {
+    const int64_t mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile;
+    const int64_t npad = (N + kH16Tile - 1) / kH16Tile * kH16Tile;
+    return (size_t)mpad * (size_t)K * 2 + (size_t)splits * (size_t)(mpad + npad) * sizeof(int);
+}
+
+int launch_gemm_h16a(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
+                     uint16_t* y, float* partial, int M, int N, int K, int splits, int groups_per_split,
+                     void* a_ws, bool rows128, hipStream_t stream) {
+    const int G = K >> 5;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 256 != 0 || splits < 1 || groups_per_split <= 0 ||
+        groups_per_split % 8 != 0 || (long long)splits * groups_per_split < G ||
+        (long long)(splits - 1) * groups_per_split >= G || (splits > 1 && partial == nullptr) || a_ws == nullptr ||
+        ((reinterpret_cast<uintptr_t>(xs) | reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(a_ws)) &
+         15u) != 0)
+        return (int)hipErrorInvalidValue;
+    const int mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile;
+    const int npad = (N + kH16Tile - 1) / kH16Tile * kH16Tile;
+    uint8_t* a16 = static_cast<uint8_t*>(a_ws);
+    int* ea = reinterpret_cast<int*>(a16 + (size_t)mpad * K * 2);
+    int* eb = ea + (size_t)splits * mpad;
+    const int mblocks = mpad / 32, nblocks = npad / 32;
+    const int chunks = (groups_per_split + kPrepChunk - 1) / kPrepChunk;
+    const long long na = (long long)mblocks * splits * chunks, nprep = na + (long long)nblocks * splits;
     const int tr = rows128 ? 128 : 256;
     const long long tiles = (long long)((N + kH16Tile - 1) / kH16Tile) * ((M + tr - 1) / tr) * splits;
-    if (rows128) {
-        gemm_h16q_kernel<4><<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K,
-                                                                        groups_per_split, splits);
-        return (int)hipGetLastError();
-    }
-    gemm_h16q_kernel<8><<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K,
-                                                                 groups_per_split, splits);
+    if (nprep > 0x7fffffffLL || tiles > 0x7fffffffLL) return (int)hipErrorInvalidValue;
+    h16_prep_kernel<<<dim3((unsigned)nprep), 256, 0, stream>>>(xq, xs, a16, ea, ws, eb, M, N, G, groups_per_split,
+                                                               mblocks, nblocks, chunks, (int)na);
+    const int e = (int)hipGetLastError();
+    if (e != 0) return e;
+    if (rows128)
+        gemm_h16q_kernel<8><<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K,
+                                                                       groups_per_split);
+    else
+        gemm_h16q_kernel<16><<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K,
+                                                                        groups_per_split);
     return (int)hipGetLastError();
 }
 

@@ -745,7 +745,7 @@ static size_t plan_bytes(const Plan& p, int64_t M, int64_t N, int64_t K) {
 #define WUSH_H16A_MIN_N 8192
 #endif
 // 64 < M <= this, where the 256-row fp16 tiles do not run: the
-// pre-converted-activation fp16 tiles with 128-row tiles (gemm_h16q_kernel<4>)
+// pre-converted-activation fp16 tiles with 128-row tiles (gemm_h16q_kernel<8>)
 // on weights of at least WUSH_H16A_MIN_N columns, when they make at least
 // WUSH_H16R_MIN_WGS workgroups, in place of the int8 tiles (0: off).
 // Measured on MI355X against the int8 tiles: L70 (K=8192, N=57344) M=128 154

@@ -308,6 +308,10 @@ __device__ __forceinline__ uint32_t lds_addr(const void* l) {
 __device__ __forceinline__ void dma16(const void* g, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(lds) : "m0");
 }
+// the same from a wave-uniform base plus a 32-bit lane offset
+__device__ __forceinline__ void dma16_uniform(const void* base, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds) : "m0");
+}
 __device__ __forceinline__ void dma4(const void* g, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(lds) : "m0");
 }
