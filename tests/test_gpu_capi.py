@@ -583,6 +583,29 @@ def test_gemm_stream_k_split_shapes(capi, M, N, K):
     assert rel_fro(y, ref) < FRO_TOL, (M, N, K, rel_fro(y, ref))
 
 
+@pytest.mark.parametrize("M,N", [(8, 1024), (8, 1023), (7, 1021), (9, 1022)])
+def test_splitk_reduce_vector_and_scalar(capi, M, N):
+    # the partials' sum, four outputs a thread where M * N and y allow it, else
+    # one: the same bits for a y of 2-byte alignment, and nothing past the end
+    import torch
+    g = rng(4285 + M + N)
+    K = 16384
+    xq, xs, wq, ws = _rand_operands(g, M, N, K)
+    d = _dev_operands(xq, xs, wq, ws)
+    wsb = capi.gemm_s4_workspace_bytes(M, N, K)
+    assert wsb > 0
+    work = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    out = []
+    for off in (0, 1):
+        buf = torch.full((M * N + 16,), 7.0, dtype=torch.float16, device="cuda")
+        capi.gemm_s4(*[t.data_ptr() for t in d], buf.data_ptr() + 2 * off, M, N, K, work.data_ptr(), wsb, _stream())
+        torch.cuda.synchronize()
+        assert (buf[:off] == 7.0).all() and (buf[off + M * N:] == 7.0).all()
+        out.append(f16_tensor_f64(buf[off:off + M * N]))
+    assert np.array_equal(out[0], out[1])
+    assert rel_fro(out[0].reshape(M, N), oracle.gemm_f64(xq, xs, wq, ws)) < FRO_TOL
+
+
 @pytest.mark.parametrize("M,N,K,groups", [
     # wide weights (4 K ways): 40 stages in runs of 10 per wavefront, so the
     # scale chunks of 4 stages start at stages 0, 4, 8 of a run, the last one
