@@ -113,17 +113,25 @@ int wush_gemv_int4_supported(int64_t M, int64_t N, int64_t K);
  * choose a plan that needs no more than it is given (same results). */
 size_t wush_gemm_s4_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
+/* Bytes of workspace with which wush_gemm_s4 runs its fastest plan; at least
+ * wush_gemm_s4_workspace_bytes, and more where that plan also converts the
+ * activations to fp16 operands on weights of fewer than 8192 rows (M > 64,
+ * K % 256 == 0, 16-byte aligned scales, from about 2^32 multiply-adds): with
+ * fewer bytes than this, wush_gemm_s4 runs the plan of
+ * wush_gemm_s4_workspace_bytes there.  The reference has no counterpart. */
+size_t wush_gemm_s4_best_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
 /* Group-scaled W4A4 GEMM, any M >= 1, K % 32 == 0: the product of
  * wush_gemv_int4, y (M, N) fp16.  On int8 MFMA with exact int32 group dots,
- * except for prefill shapes (K % 256 == 0, M > 128, at least 64 tiles of
- * 256x256 or N >= 2048, and at least 128 workgroups counting the K slices of
- * at least 32 groups each that the workspace holds from M = 512), for
- * 64 < M <= 256 with N >= 8192 when the workspace holds the converted
- * activations (128-row tiles, at least 192 workgroups with at most 2 K slices
- * of at least 64 groups), and for 32 < M <= 64 with 49953 <= N <= 57344 and
- * K % 1024 == 0 (16-byte aligned codes and scales), which run fp16 MFMA on
- * code*scale operands (exact after
- * a power-of-two shift per row and column) accumulated in fp32 over all of K.
+ * except for three ranges that run fp16 MFMA on code*scale operands (exact
+ * after a power-of-two shift per row and column) accumulated in fp32 over all
+ * of K: M > 64 with K % 256 == 0, from about 2^32 multiply-adds (3e9; 4.8e9 for
+ * N < 2048; 192 tiles of 128 x 256 outputs at N >= 8192), when the workspace
+ * holds the converted activations (see the two functions above); without that
+ * room M > 128 with K % 256 == 0, at least 64 tiles of 256x256 or N >= 2048, and
+ * at least 128 workgroups counting the K slices of at least 32 groups each
+ * that the workspace holds from M = 512; and 32 < M <= 64 with 49953 <= N <=
+ * 57344 and K % 1024 == 0 (16-byte aligned codes and scales).
  * Both agree with the fp64 product to 2e-3 relative Frobenius (tested); a row
  * or column with a non-finite scale gives NaN there.
  * Replaces w4a4_gemm_s4 (csrc/gemm_s4.cu:320-379) and the superseded

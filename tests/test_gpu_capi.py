@@ -932,11 +932,12 @@ def test_gemm_h16_nonfinite_scales(capi, M, N):
     assert rel_fro(got, ref) < FRO_TOL, rel_fro(got, ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(515, 8195, 2048),     # K split in 2: scalar fp32 partial stores
-                                   (513, 8198, 2048),     # ... rows of 4-byte alignment
+@pytest.mark.parametrize("M,N,K", [(203, 8195, 8192),     # K split: scalar fp32 partial stores
+                                   (131, 8198, 8192),     # ... rows of 4-byte alignment
+                                   (130, 8196, 6144),     # ... 16-byte partial stores, fp16 rows of 8 bytes
                                    (129, 33001, 256),     # one double batch, scalar fp16 stores
                                    (257, 32772, 768),     # a one-row second tile, 8-byte rows
-                                   (65, 49155, 512)])     # 128-row tiles, scalar fp16 stores
+                                   (65, 49155, 512)])     # scalar fp16 stores
 def test_gemm_h16q_ragged_columns(capi, M, N, K):
     # converted-activation tiles whose rows of y are not whole 16-byte chunks,
     # with a non-finite row and a non-finite last column (split plans write
@@ -955,6 +956,44 @@ def test_gemm_h16q_ragged_columns(capi, M, N, K):
     A = _abs_product(xq[rows], xs[rows], wq[cols], ws[cols])
     bound = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64) + 2 * K * 2.0 ** -24 * A + 2.0 ** -25
     assert (np.abs(got - ref) <= bound).all(), (M, N, K, float((np.abs(got - ref) / bound).max()))
+
+
+# Narrow weights (N < 8192): every tile height (64, 128, 256 rows) and K splits
+# from 1 to 16, ragged M and N, G = K / 32 that splits by 8 only once
+@pytest.mark.parametrize("M,N,K", [(65, 4096, 16384), (256, 4096, 4096), (512, 4099, 4096), (129, 6146, 6144),
+                                   (1000, 2051, 2304), (1030, 4096, 2048), (2047, 4100, 2048), (4090, 4104, 512),
+                                   (400, 1027, 14336), (70, 8190, 8192)])
+def test_gemm_best_workspace_plan_agrees(capi, M, N, K):
+    # the converted-activation plan, taken from
+    # wush_gemm_s4_best_workspace_bytes on, and the plan of the bytes that
+    # wush_gemm_s4_workspace_bytes names (one byte less than best keeps it):
+    # both within one fp16 rounding plus 2K rounded fp32 additions of the fp64
+    # product; a row and a column with a NaN scale are NaN in both
+    import torch
+    g = rng(4950 + M)
+    xq, xs, wq, ws = _rand_operands(g, M, N, K)
+    xs[2, 1], ws[N - 2, 0] = 0x7FC0, 0x7FC0
+    d = _dev_operands(xq, xs, wq, ws)
+    base, best = capi.gemm_s4_workspace_bytes(M, N, K), capi.gemm_s4_best_workspace_bytes(M, N, K)
+    assert best > base and best >= 2 * M * K
+    work = torch.full((best,), 0xFF, dtype=torch.uint8, device="cuda")
+    rows = np.array([r for r in _sample(g, M, 24) if r != 2])
+    cols = np.array([c for c in _sample(g, N, 500) if c != N - 2])
+    ref = oracle.gemm_f64(xq[rows], xs[rows], wq[cols], ws[cols])
+    A = _abs_product(xq[rows], xs[rows], wq[cols], ws[cols])
+    bound = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64) + 2 * K * 2.0 ** -24 * A + 2.0 ** -25
+    ys = []
+    for wsb in (best, best - 1, base):
+        y = torch.empty(M, N, dtype=torch.float16, device="cuda")
+        capi.gemm_s4(*[t.data_ptr() for t in d], y.data_ptr(), M, N, K, work.data_ptr() if wsb else None, wsb,
+                     _stream())
+        torch.cuda.synchronize()
+        ys.append(f16_tensor_f64(y))
+        assert np.isnan(ys[-1][2]).all() and np.isnan(ys[-1][:, N - 2]).all()
+        assert np.isfinite(np.delete(np.delete(ys[-1], 2, axis=0), N - 2, axis=1)).all()
+        got = ys[-1][np.ix_(rows, cols)]
+        assert (np.abs(got - ref) <= bound).all(), (M, N, K, wsb, float((np.abs(got - ref) / bound).max()))
+    assert np.array_equal(np.nan_to_num(ys[1]), np.nan_to_num(ys[2]))
 
 
 # Shapes the planner sends to the fp16-MFMA streaming kernel (gemm_h16s:

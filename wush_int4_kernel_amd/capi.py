@@ -25,6 +25,7 @@ SIGNATURES = {
     "wush_gemv_int4": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _I),
     "wush_gemv_int4_supported": ([_I64, _I64, _I64], _I),
     "wush_gemm_s4_workspace_bytes": ([_I64, _I64, _I64], _SZ),
+    "wush_gemm_s4_best_workspace_bytes": ([_I64, _I64, _I64], _SZ),
     "wush_gemm_s4": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _SZ, _P], _I),
     "wush_gemm_s4_noalloc": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _I),
     "wush_mfma_selftest": ([_P, _P, _P, _P], _I),
@@ -80,6 +81,10 @@ def gemv_int4_supported(M, N, K) -> bool:
 
 def gemm_s4_workspace_bytes(M, N, K) -> int:
     return int(load().wush_gemm_s4_workspace_bytes(M, N, K))
+
+
+def gemm_s4_best_workspace_bytes(M, N, K) -> int:
+    return int(load().wush_gemm_s4_best_workspace_bytes(M, N, K))
 
 
 def gemm_s4(xq, xs, wq, ws, y, M, N, K, workspace, workspace_bytes, stream) -> None:

@@ -130,9 +130,20 @@ torch::Tensor product_2d(const torch::Tensor& xq2, const torch::Tensor& xs2, con
                      op);
         return y;
     }
-    const size_t wsb = wush_gemm_s4_workspace_bytes(M, N, K);
+    size_t wsb = wush_gemm_s4_best_workspace_bytes(M, N, K);
+    const auto bytes = torch::dtype(torch::kUInt8).device(xq2.device());
     torch::Tensor work;
-    if (wsb) work = torch::empty({(int64_t)wsb}, torch::dtype(torch::kUInt8).device(xq2.device()));
+    if (wsb) {
+        // without room for the fastest plan's workspace, the smaller one's
+        try {
+            work = torch::empty({(int64_t)wsb}, bytes);
+        } catch (const c10::OutOfMemoryError&) {
+            const size_t less = wush_gemm_s4_workspace_bytes(M, N, K);
+            if (less == wsb) throw;
+            wsb = less;
+            if (wsb) work = torch::empty({(int64_t)wsb}, bytes);
+        }
+    }
     check_status(wush_gemm_s4(ptr<uint8_t>(xq2), ptr<uint16_t>(xs2), ptr<uint8_t>(wq), ptr<uint16_t>(ws),
                               ptr<uint16_t>(y), M, N, K, wsb ? work.data_ptr() : nullptr, wsb,
                               current_stream(xq2)),

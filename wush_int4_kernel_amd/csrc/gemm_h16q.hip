@@ -470,10 +470,11 @@ size_t gemm_h16a_workspace_bytes(int64_t M, int64_t N, int64_t K, int splits) {
 
 int launch_gemm_h16a(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
                      uint16_t* y, float* partial, int M, int N, int K, int splits, int groups_per_split,
-                     void* a_ws, bool rows128, hipStream_t stream) {
+                     void* a_ws, int tile_rows, hipStream_t stream) {
     const int G = K >> 5;
     if (M <= 0 || N <= 0 || K <= 0 || K % 256 != 0 || splits < 1 || groups_per_split <= 0 ||
         groups_per_split % 8 != 0 || (long long)splits * groups_per_split < G ||
+        (tile_rows != 64 && tile_rows != 128 && tile_rows != 256) ||
         (long long)(splits - 1) * groups_per_split >= G || (splits > 1 && partial == nullptr) || a_ws == nullptr ||
         ((reinterpret_cast<uintptr_t>(xs) | reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(a_ws)) &
          15u) != 0)
@@ -486,19 +487,14 @@ int launch_gemm_h16a(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, c
     const int mblocks = mpad / 32, nblocks = npad / 32;
     const int chunks = (groups_per_split + kPrepChunk - 1) / kPrepChunk;
     const long long na = (long long)mblocks * splits * chunks, nprep = na + (long long)nblocks * splits;
-    const int tr = rows128 ? 128 : 256;
-    const long long tiles = (long long)((N + kH16Tile - 1) / kH16Tile) * ((M + tr - 1) / tr) * splits;
+    const long long tiles = (long long)((N + kH16Tile - 1) / kH16Tile) * ((M + tile_rows - 1) / tile_rows) * splits;
     if (nprep > 0x7fffffffLL || tiles > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     h16_prep_kernel<<<dim3((unsigned)nprep), 256, 0, stream>>>(xq, xs, a16, ea, ws, eb, M, N, G, groups_per_split,
                                                                mblocks, nblocks, chunks, (int)na);
     const int e = (int)hipGetLastError();
     if (e != 0) return e;
-    if (rows128)
-        gemm_h16q_kernel<8><<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K,
-                                                                       groups_per_split);
-    else
-        gemm_h16q_kernel<16><<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K,
-                                                                        groups_per_split);
+    const auto kernel = tile_rows == 64 ? gemm_h16q_kernel<4> : tile_rows == 128 ? gemm_h16q_kernel<8> : gemm_h16q_kernel<16>;
+    kernel<<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K, groups_per_split);
     return (int)hipGetLastError();
 }
 

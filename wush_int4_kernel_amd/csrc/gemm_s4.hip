@@ -24,6 +24,8 @@
 // conflict-free.  Skinny M uses split-K: each K slice writes fp32 partials to
 // a caller-provided workspace and a second kernel sums the slices in a fixed
 // order (deterministic, graph-capturable, no atomics, no memset).
+#include <algorithm>
+
 #include "wush_device.h"
 #include "gemm_h16.h"
 #include "setup.h"
@@ -755,37 +757,34 @@ static size_t plan_bytes(const Plan& p, int64_t M, int64_t N, int64_t K) {
 #ifndef WUSH_H16_SPLIT_MIN_M
 #define WUSH_H16_SPLIT_MIN_M 512
 #endif
-// Pre-converted activations (gemm_h16q.hip) when the weights have at least this
-// many columns, the scales are 16-byte aligned and the workspace has room
-// for M x K x 2 bytes more.
+// Converted-activation fp16 tiles (gemm_h16q.hip), M > 64, K % 256 == 0,
+// 16-byte aligned scales and room in the workspace.  They cost three launches
+// (conversion, GEMM, split-K sum) where the int8 tiles cost one or two, so
+// they take over from this many multiply-adds: M=N=4096-wide K=4096 at M=256
+// (2^32) 30.5 -> 27.3 us, at M=128 20.5 -> 25.4; 300 x 9000 x 1536 (0.97 of 2^32)
+// 26.8 -> 22.0, 70 x 8192 x 4096 (0.55) 24.7 -> 23.8, 250 x 8192 x 1024 (0.49)
+// 14.3 -> 17.1.  On fewer columns than WUSH_H16A_NARROW_N the int8 tiles hold
+// out longer: 4000 x 512 x 2048 (0.98) 28.4 -> 30.4, 600 x 1024 x 8192 (1.17)
+// 37.3 -> 32.5.
+#ifndef WUSH_H16A_MIN_WORK
+#define WUSH_H16A_MIN_WORK 3000000000
+#endif
+#ifndef WUSH_H16A_NARROW_N
+#define WUSH_H16A_NARROW_N 2048
+#endif
+#ifndef WUSH_H16A_NARROW_MIN_WORK
+#define WUSH_H16A_NARROW_MIN_WORK 4800000000
+#endif
+// ... and below it where this many 128-row tiles come without a K split
+// (short K on wide weights): 1000 x 8192 x 256 18.6 -> 13.9 us.
+#ifndef WUSH_H16A_MIN_TILES
+#define WUSH_H16A_MIN_TILES 192
+#endif
+// On weights narrower than this the plan is taken only with a workspace of
+// wush_gemm_s4_best_workspace_bytes: wush_gemm_s4_workspace_bytes keeps
+// naming the smaller one of the per-tile and int8 plans there.
 #ifndef WUSH_H16A_MIN_N
 #define WUSH_H16A_MIN_N 8192
-#endif
-// 64 < M <= this, where the 256-row fp16 tiles do not run: the
-// pre-converted-activation fp16 tiles with 128-row tiles (gemm_h16q_kernel<8>)
-// on weights of at least WUSH_H16A_MIN_N columns, when they make at least
-// WUSH_H16R_MIN_WGS workgroups, in place of the int8 tiles (0: off).
-// Measured on MI355X against the int8 tiles: L70 (K=8192, N=57344) M=128 154
-// vs 254 us, M=96 156 vs 248, M=72 147 vs 225, K=8192 N=28672 M=128 95 vs 134;
-// K=4096 N=24576 M=128 (2 K slices) 59.7 vs 67.9.  With 4 slices it was not
-// a steady gain (K=N=8192 M=128: 47.4 vs 49.8 on one box, 56.2 vs 52.3 on
-// another), and with slices of 32 groups (K=4096 N=8192) it took 40.2
-// against 32.0: hence at most 2 slices of at least 64 groups.  Above M = 128
-// (256-row tiles too few): K=4096 N=24576 M=256 74.9 vs 111.4, M=192 73.1 vs
-// 102.8, K=4096 N=16384 M=200 (2 slices) 61.6 vs 75.4; with 128 workgroups
-// it lost (K=N=8192 M=256 83.7 vs 81.3, M=192 79.5 vs 66.2; K=4096 N=8192
-// M=256 54.8 vs 50.2), hence at least 192.
-#ifndef WUSH_H16R_MAX_M
-#define WUSH_H16R_MAX_M 256
-#endif
-#ifndef WUSH_H16R_MIN_WGS
-#define WUSH_H16R_MIN_WGS 192
-#endif
-#ifndef WUSH_H16R_MIN_SPLIT_GROUPS
-#define WUSH_H16R_MIN_SPLIT_GROUPS 64
-#endif
-#ifndef WUSH_H16R_MAX_SPLITS
-#define WUSH_H16R_MAX_SPLITS 2
 #endif
 // 8 < M <= 64 streaming kernel (gemm_s4_stream32_kernel).  K ways: 4
 // wavefronts per workgroup on wide weights, 8 on narrow ones (measured on
@@ -823,10 +822,64 @@ constexpr int kStream32MaxM = WUSH_S32_MAXM;
 constexpr int stream32_kw(int64_t n) { return n > WUSH_S32_WIDE_N ? WUSH_S32_KW_WIDE : WUSH_S32_KW_NARROW; }
 constexpr int kStream32Waves = WUSH_S32_WAVES;
 
+// Whether the converted-activation fp16 tiles run (M, N, K), given the room.
+static bool h16a_preferred(int64_t M, int64_t N, int64_t K) {
+    if (K % 256 != 0 || M <= 64) return false;
+    const double work = (double)M * (double)N * (double)K;
+    if (work >= (N < WUSH_H16A_NARROW_N ? (double)WUSH_H16A_NARROW_MIN_WORK : (double)WUSH_H16A_MIN_WORK)) return true;
+    return N >= WUSH_H16A_MIN_N && ((M + 127) / 128) * ((N + 255) / 256) >= WUSH_H16A_MIN_TILES;
+}
+
+// Estimated us of the converted-activation tiles with `rows`-row tiles and s
+// K slices: 5 for the launches, then per round of up to 256 workgroups (one
+// per CU) a fixed cost (ring fill, epilogue) and a cost per 32-wide stage that
+// grows with the workgroups running (`lo` alone, `hi` with the chip full: the
+// clock follows the power), the conversion's bytes at 5 TB/s, and for s > 1
+// the partials' write, read and launch.  Fitted to 64 shapes (64 <= M <= 4096,
+// 512 <= N <= 65536, 256 <= K <= 16384, every tile height and K split): the
+// tile and split with the least estimate is on average 0.7% slower than the
+// best one measured, 10% at worst.
+static double h16a_cost_us(int64_t M, int64_t N, int64_t K, int rows, int s) {
+    static const struct { int rows; double fixed, lo, hi; } kCost[] = {
+        {64, 3.5, 0.225, 0.275}, {128, 4.5, 0.3125, 0.40}, {256, 8.0, 0.50, 0.66}};
+    const auto& c = kCost[rows == 64 ? 0 : rows == 128 ? 1 : 2];
+    const int64_t wgs = ((M + rows - 1) / rows) * ((N + 255) / 256) * s;
+    const double stages = (double)(K / 32) / s;
+    auto round_us = [&](int64_t n) { return n ? c.fixed + stages * (c.lo + (c.hi - c.lo) * (double)n / 256.0) : 0.0; };
+    double us = 5.0 + (double)(wgs / 256) * round_us(256) + round_us(wgs % 256);
+    us += (2.5 * (double)M * (double)K + (double)N * (double)K / 16.0) / 5e6;
+    if (s > 1) us += 4.5 + 0.22e-6 * 4.0 * s * (double)M * (double)N;
+    return us;
+}
+
+// The cheapest tile height and K split (slices of whole 8-group blocks) whose
+// workspace fits `room`; false if none does.
+static bool plan_h16a(int64_t M, int64_t N, int64_t K, size_t room, Plan* out) {
+    const int64_t G = K / 32;
+    double best = 0.0;
+    bool found = false;
+    for (int rows = 64; rows <= 256; rows *= 2) {
+        if (rows > 64 && M <= rows / 2) break;
+        for (int s = 1; s <= 16 && G % (8 * s) == 0; s *= 2) {
+            Plan q;
+            q.cfg = 5; q.mr = 32; q.tm = rows; q.tn = 256; q.sg = 1;
+            q.splits = s;
+            q.groups_per_split = (int)(G / s);
+            q.a16 = true;
+            if (plan_bytes(q, M, N, K) > room) break;
+            const double us = h16a_cost_us(M, N, K, rows, s);
+            if (!found || us < best) { *out = q; best = us; found = true; }
+        }
+    }
+    return found;
+}
+
 // scales16: both scale tensors (and both code tensors) are 16-byte aligned
 // (the streaming kernels read them 16 bytes at a time).
+// allow_a16: converted activations may go to the workspace; narrow_a16: also
+// for weights narrower than WUSH_H16A_MIN_N.
 static Plan make_plan(int64_t M, int64_t N, int64_t K, size_t ws_bytes_available, bool allow_split,
-                      bool scales16, bool allow_a16 = true) {
+                      bool scales16, bool allow_a16, bool narrow_a16) {
     Plan p;
     p.mr = 32;
     const int64_t G0 = K / 32;
@@ -861,6 +914,10 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, size_t ws_bytes_available
         p.groups_per_split = (int)gps;
         return p;
     }
+    if (allow_split && allow_a16 && scales16 && (narrow_a16 || N >= WUSH_H16A_MIN_N) && h16a_preferred(M, N, K)) {
+        Plan q;
+        if (plan_h16a(M, N, K, ws_bytes_available, &q)) return q;
+    }
     if (allow_split && K % 256 == 0 && M >= WUSH_H16_MIN_M &&
         (((M + 255) / 256) * ((N + 255) / 256) >= WUSH_H16_FEW_TILES || N >= WUSH_H16_FEW_TILES_MIN_N)) {
         // fp16-MFMA tiles, with K split across workgroups (slices of a
@@ -875,31 +932,8 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, size_t ws_bytes_available
             p.cfg = 5; p.tm = 256; p.tn = 256; p.sg = 1;
             p.splits = s;
             p.groups_per_split = (int)(G0 / s);
-            if (allow_a16 && scales16 && N >= WUSH_H16A_MIN_N) {
-                Plan q = p;
-                q.a16 = true;
-                if (plan_bytes(q, M, N, K) <= ws_bytes_available) p.a16 = true;
-            }
             return p;
         }
-    }
-    if (allow_split && allow_a16 && scales16 && K % 256 == 0 && M > 64 && M <= WUSH_H16R_MAX_M &&
-        N >= WUSH_H16A_MIN_N) {
-        // 128-row fp16 tiles (where the 256-row ones do not run), K split
-        // while twice the workgroups still run in one round on 256 CUs (one
-        // workgroup per CU fits)
-        const int64_t tiles = ((M + 127) / 128) * ((N + 255) / 256);
-        int s = 1;
-        while (s < WUSH_H16R_MAX_SPLITS && tiles * 2 * s <= 256 && G0 % (16 * s) == 0 &&
-               G0 / (2 * s) >= WUSH_H16R_MIN_SPLIT_GROUPS &&
-               (size_t)(2 * s) * (size_t)M * (size_t)N * sizeof(float) <= ws_bytes_available)
-            s *= 2;
-        Plan q = p;
-        q.cfg = 5; q.tm = 128; q.tn = 256; q.sg = 1;
-        q.splits = s;
-        q.groups_per_split = (int)(G0 / s);
-        q.a16 = true;
-        if (tiles * s >= WUSH_H16R_MIN_WGS && plan_bytes(q, M, N, K) <= ws_bytes_available) return q;
     }
     const int64_t big_tiles = ((M + 32 * WUSH_PF_BM * 2 - 1) / (32 * WUSH_PF_BM * 2)) *
                               ((N + 32 * WUSH_PF_BN * 2 - 1) / (32 * WUSH_PF_BN * 2));
@@ -929,6 +963,20 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, size_t ws_bytes_available
     p.splits = s;
     p.groups_per_split = (int)gps;
     return p;
+}
+
+static size_t base_bytes(int64_t M, int64_t N, int64_t K) {
+    return plan_bytes(make_plan(M, N, K, (size_t)-1, true, true, true, false), M, N, K);
+}
+
+// Workspace bytes of wush_gemm_s4: `base` as wush_gemm_s4_workspace_bytes
+// reports it, and the larger number from which the converted-activation plan
+// runs on narrow weights too.  It is always above `base` where the plans
+// differ, so that a caller with `base` bytes keeps that plan and its bits.
+static size_t best_bytes(int64_t M, int64_t N, int64_t K, size_t base) {
+    const Plan p = make_plan(M, N, K, (size_t)-1, true, true, true, true);
+    const size_t b = plan_bytes(p, M, N, K);
+    return p.a16 && N < WUSH_H16A_MIN_N ? std::max(b, base + 256) : base;
 }
 
 template <int BM, int BN, int WM, int WN, int SG, int MR, bool PT>
@@ -970,7 +1018,11 @@ static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, co
                             reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
     // the pre-converted activations need a 16-byte aligned workspace
     allow_a16 = allow_a16 && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
-    const Plan p = make_plan(M, N, K, workspace ? ws_bytes : 0, !PT, scales16, allow_a16);
+    const size_t room = workspace ? ws_bytes : 0;
+    bool narrow_a16 = false;
+    if (!PT && allow_a16 && N < WUSH_H16A_MIN_N && room > 0 && h16a_preferred(M, N, K))
+        narrow_a16 = room >= best_bytes(M, N, K, base_bytes(M, N, K));
+    const Plan p = make_plan(M, N, K, room, !PT, scales16, allow_a16, narrow_a16);
     WUSH_REQUIRE((N + p.tn - 1) / p.tn <= 0x7fffffffLL && (M + p.tm - 1) / p.tm <= 65535);
     float* partial = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     const int m = (int)M, n = (int)N, k = (int)K;
@@ -982,7 +1034,7 @@ static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, co
             uint8_t* wsp = static_cast<uint8_t*>(workspace);
             const int st = p.a16 ? launch_gemm_h16a(xq, xs, wq, ws, y, partial, m, n, k, p.splits,
                                                     p.groups_per_split, wsp + plan_a16_offset(p, M, N),
-                                                    p.tm == 128, stream)
+                                                    p.tm, stream)
                                  : launch_gemm_h16(xq, xs, wq, ws, y, partial, m, n, k, p.splits,
                                                    p.groups_per_split, stream);
             if (st != 0 || p.splits == 1) return st;
@@ -1026,8 +1078,12 @@ extern "C" {
 
 size_t wush_gemm_s4_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 32) return 0;
-    const wush::Plan p = wush::make_plan(M, N, K, (size_t)-1, true, true);
-    return wush::plan_bytes(p, M, N, K);
+    return wush::base_bytes(M, N, K);
+}
+
+size_t wush_gemm_s4_best_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 32) return 0;
+    return wush::best_bytes(M, N, K, wush::base_bytes(M, N, K));
 }
 
 int wush_gemm_s4(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
@@ -1059,7 +1115,7 @@ int wush_gemm_s4_noalloc(const uint8_t* xq, const uint16_t* xs, const uint8_t* w
     const bool scales16 = ((reinterpret_cast<uintptr_t>(xs) | reinterpret_cast<uintptr_t>(ws) |
                             reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
     const size_t cap = (size_t)WUSH_GEMM_SCRATCH_BYTES;
-    const size_t need = wush::plan_bytes(wush::make_plan(M, N, K, cap, true, scales16, false), M, N, K);
+    const size_t need = wush::plan_bytes(wush::make_plan(M, N, K, cap, true, scales16, false, false), M, N, K);
     if (need > cap) return WUSH_ERROR_SCRATCH_TOO_SMALL;
     int dev = 0;
     const int st = wush::device_setup(&dev);
