@@ -6,6 +6,7 @@
 // (include/wush_int4.h).  No computation happens here.
 #include <torch/extension.h>
 
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
@@ -28,10 +29,25 @@ T* ptr(const torch::Tensor& t) {
     return reinterpret_cast<T*>(t.data_ptr());
 }
 
-std::vector<int64_t> with_last(const torch::Tensor& t, int64_t last) {
-    std::vector<int64_t> s = t.sizes().vec();
+c10::SmallVector<int64_t, 6> with_last(const torch::Tensor& t, int64_t last) {
+    c10::SmallVector<int64_t, 6> s(t.sizes().begin(), t.sizes().end());
     s.back() = last;
     return s;
+}
+
+// Uninitialized contiguous tensor on t's device, straight from the caching
+// allocator: every op here writes its outputs whole.  torch::empty goes
+// through the dispatcher, 1.7 us a tensor against 3.3 us for a kernel launch;
+// with it and views of flat outputs an eager M=1 K=N=4096 layer step (two
+// launches) took 11.6 us of host time, without 8.2.
+torch::Tensor new_tensor(c10::IntArrayRef sizes, at::ScalarType dtype, const torch::Tensor& t) {
+    return torch::Tensor(at::detail::empty_cuda(sizes, dtype, t.device(), std::nullopt));
+}
+
+// t as (rows, last), without a dispatched reshape where it is that already.
+torch::Tensor as_rows(const torch::Tensor& t, int64_t last) {
+    if (t.dim() == 2 && last > 0 && t.size(1) == last) return t;
+    return t.reshape({-1, last});
 }
 
 // quant_int4 (csrc/quant_int4.cu:109-134).  Also accepts fp16/fp32 input,
@@ -44,13 +60,13 @@ std::vector<torch::Tensor> quant_int4(torch::Tensor x) {
     TORCH_CHECK(x.dim() >= 1 && x.size(-1) % 32 == 0, "last dim must be multiple of 32");
     const at::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
     const int64_t n_groups = x.numel() / 32;
-    auto q = torch::empty({x.numel() / 2}, torch::dtype(torch::kUInt8).device(x.device()));
-    auto s = torch::empty({n_groups}, torch::dtype(torch::kBFloat16).device(x.device()));
+    auto q = new_tensor(with_last(x, x.size(-1) / 2), torch::kUInt8, x);
+    auto s = new_tensor(with_last(x, x.size(-1) / 32), torch::kBFloat16, x);
     const int code = dt == torch::kBFloat16 ? WUSH_DTYPE_BF16 : (dt == torch::kHalf ? WUSH_DTYPE_F16 : WUSH_DTYPE_F32);
     check_status(wush_quant_int4(x.data_ptr(), code, ptr<uint8_t>(q), ptr<uint16_t>(s), n_groups,
                                  current_stream(x)),
                  "quant_int4");
-    return {q.view(with_last(x, x.size(-1) / 2)), s.view(with_last(x, x.size(-1) / 32))};
+    return {q, s};
 }
 
 // fused_transform_quant_int4 and its variants (csrc/fused_tq_int4.cu:87-118,
@@ -69,12 +85,12 @@ std::vector<torch::Tensor> fused_tq_impl(torch::Tensor x, torch::Tensor t, bool 
     const int64_t rows = K ? x.numel() / K : 0;
     if (need_rows) TORCH_CHECK(rows >= 1, "rows must be >= 1");
     const at::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
-    auto q = torch::empty({rows * C * 16}, torch::dtype(torch::kUInt8).device(x.device()));
-    auto s = torch::empty({rows * C}, torch::dtype(torch::kBFloat16).device(x.device()));
+    auto q = new_tensor(with_last(x, K / 2), torch::kUInt8, x);
+    auto s = new_tensor(with_last(x, C), torch::kBFloat16, x);
     check_status(wush_fused_tq(ptr<uint16_t>(x), ptr<uint16_t>(t), ptr<uint8_t>(q), ptr<uint16_t>(s),
                                rows, K, current_stream(x)),
                  "fused_transform_quant_int4");
-    return {q.view(with_last(x, K / 2)), s.view(with_last(x, C))};
+    return {q, s};
 }
 
 std::vector<torch::Tensor> fused_transform_quant_int4(torch::Tensor x, torch::Tensor t) {
@@ -118,12 +134,14 @@ bool gemv_preferred(int64_t M, int64_t N, int64_t K) {
     return wush_gemv_int4_supported(M, N, K) != 0 && (M <= 4 || N > 32768);
 }
 
-// Shared product launch: y (M, N) fp16 = group-scaled product.
+// Shared product launch: y (M, N) fp16 = group-scaled product, in `sizes`
+// (default (M, N)).
 torch::Tensor product_2d(const torch::Tensor& xq2, const torch::Tensor& xs2, const torch::Tensor& wq,
-                         const torch::Tensor& ws, int64_t K, const char* op) {
+                         const torch::Tensor& ws, int64_t K, const char* op, c10::IntArrayRef sizes = {}) {
     const int64_t M = xq2.size(0), N = wq.size(0);
     const at::hip::OptionalHIPGuardMasqueradingAsCUDA guard(xq2.device());
-    auto y = torch::empty({M, N}, torch::dtype(torch::kHalf).device(xq2.device()));
+    const int64_t mn[2] = {M, N};
+    auto y = new_tensor(sizes.empty() ? c10::IntArrayRef(mn, 2) : sizes, torch::kHalf, xq2);
     if (gemv_preferred(M, N, K)) {
         check_status(wush_gemv_int4(ptr<uint8_t>(xq2), ptr<uint16_t>(xs2), ptr<uint8_t>(wq), ptr<uint16_t>(ws),
                                     ptr<uint16_t>(y), M, N, K, current_stream(xq2)),
@@ -131,17 +149,16 @@ torch::Tensor product_2d(const torch::Tensor& xq2, const torch::Tensor& xs2, con
         return y;
     }
     size_t wsb = wush_gemm_s4_best_workspace_bytes(M, N, K);
-    const auto bytes = torch::dtype(torch::kUInt8).device(xq2.device());
     torch::Tensor work;
     if (wsb) {
         // without room for the fastest plan's workspace, the smaller one's
         try {
-            work = torch::empty({(int64_t)wsb}, bytes);
+            work = new_tensor({(int64_t)wsb}, torch::kUInt8, xq2);
         } catch (const c10::OutOfMemoryError&) {
             const size_t less = wush_gemm_s4_workspace_bytes(M, N, K);
             if (less == wsb) throw;
             wsb = less;
-            if (wsb) work = torch::empty({(int64_t)wsb}, bytes);
+            if (wsb) work = new_tensor({(int64_t)wsb}, torch::kUInt8, xq2);
         }
     }
     check_status(wush_gemm_s4(ptr<uint8_t>(xq2), ptr<uint16_t>(xs2), ptr<uint8_t>(wq), ptr<uint16_t>(ws),
@@ -157,8 +174,8 @@ torch::Tensor w4a4_gemm_s4(torch::Tensor xq, torch::Tensor xs, torch::Tensor wq,
     const int64_t K2 = xq.size(-1);
     const int64_t K = K2 * 2, G = K / 32;
     TORCH_CHECK(K % 64 == 0, "K must be multiple of 64");
-    auto xq2 = xq.reshape({-1, K2});
-    auto xs2 = xs.reshape({-1, G});
+    auto xq2 = as_rows(xq, K2);
+    auto xs2 = as_rows(xs, G);
     TORCH_CHECK(wq.dim() == 2 && wq.size(1) == K2 && ws.size(-1) == G && ws.numel() == wq.size(0) * G,
                 "K mismatch");
     TORCH_CHECK(xs2.size(0) == xq2.size(0), "K mismatch");
@@ -185,7 +202,7 @@ torch::Tensor w4a4_gemm_v1(torch::Tensor xq, torch::Tensor xs, torch::Tensor wq,
     const int64_t K2 = xq.size(-1);
     const int64_t K = K2 * 2, G = K / 32;
     TORCH_CHECK(K % 32 == 0 && wq.dim() == 2 && wq.size(1) == K2 && ws.size(-1) == G, "K mismatch");
-    return product_2d(xq.reshape({-1, K2}), xs.reshape({-1, G}), wq, ws, K, "w4a4_gemm_v1");
+    return product_2d(as_rows(xq, K2), as_rows(xs, G), wq, ws, K, "w4a4_gemm_v1");
 }
 
 // w4a4_gemm_v2 (csrc/gemm_wmma2.cu:141-181): y (M, N), K % 64 == 0.
@@ -195,7 +212,7 @@ torch::Tensor w4a4_gemm_v2(torch::Tensor xq, torch::Tensor xs, torch::Tensor wq,
     const int64_t K = K2 * 2, G = K / 32;
     TORCH_CHECK(K % 64 == 0, "K must be multiple of 64");
     TORCH_CHECK(wq.dim() == 2 && wq.size(1) == K2 && ws.size(-1) == G, "K mismatch");
-    return product_2d(xq.reshape({-1, K2}), xs.reshape({-1, G}), wq, ws, K, "w4a4_gemm_v2");
+    return product_2d(as_rows(xq, K2), as_rows(xs, G), wq, ws, K, "w4a4_gemm_v2");
 }
 
 // w4a4_gemv (csrc/gemv_int4.cu:191-223): single row, y (N,) fp16.
@@ -206,8 +223,11 @@ torch::Tensor w4a4_gemv(torch::Tensor xq, torch::Tensor xs, torch::Tensor wq, to
     const int64_t K = K2 * 2, G = K / 32;
     TORCH_CHECK(K % 32 == 0 && wq.dim() == 2 && wq.size(1) == K2 && ws.size(-1) == G && xs.numel() == G,
                 "K mismatch");
-    auto y = product_2d(xq.reshape({1, K2}), xs.reshape({1, G}), wq, ws, K, "w4a4_gemv");
-    return y.view({wq.size(0)});
+    const int64_t n[1] = {wq.size(0)};
+    auto row = [](const torch::Tensor& t, int64_t last) {
+        return t.dim() == 2 && t.size(0) == 1 && t.size(1) == last ? t : t.reshape({1, last});
+    };
+    return product_2d(row(xq, K2), row(xs, G), wq, ws, K, "w4a4_gemv", c10::IntArrayRef(n, 1));
 }
 
 // w4a4_gemv_multi (csrc/gemv_int4.cu:145-189): 1 <= M <= 8, y (M, N) fp16.
@@ -215,8 +235,8 @@ torch::Tensor w4a4_gemv_multi(torch::Tensor xq, torch::Tensor xs, torch::Tensor 
     check_packed(xq, xs, wq, ws);
     const int64_t K2 = xq.size(-1);
     const int64_t K = K2 * 2, G = K / 32;
-    auto xq2 = xq.reshape({-1, K2});
-    auto xs2 = xs.reshape({-1, G});
+    auto xq2 = as_rows(xq, K2);
+    auto xs2 = as_rows(xs, G);
     const int64_t M = xq2.size(0);
     TORCH_CHECK(M >= 1 && M <= 8, "gemv_multi expects 1<=M<=8");
     TORCH_CHECK(K % 32 == 0 && wq.dim() == 2 && wq.size(1) == K2 && ws.size(-1) == G && xs2.size(0) == M,
@@ -244,7 +264,7 @@ torch::Tensor quant_int4_tensor_scale(torch::Tensor x, double scale) {
                 "x must be contiguous CUDA bf16");
     TORCH_CHECK(x.numel() % 32 == 0, "numel must be multiple of 32");
     const at::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
-    auto q = torch::empty({x.numel() / 2}, torch::dtype(torch::kUInt8).device(x.device()));
+    auto q = new_tensor({x.numel() / 2}, torch::kUInt8, x);
     const float inv = (float)(1.0 / scale);
     check_status(wush_quant_int4_tensor_scale(ptr<uint16_t>(x), ptr<uint8_t>(q), x.numel(), inv, nullptr,
                                               current_stream(x)),
@@ -261,7 +281,7 @@ torch::Tensor quant_int4_tensor_scale_dev(torch::Tensor x, torch::Tensor inv_sca
                     inv_scale.is_contiguous() && inv_scale.numel() == 1,
                 "inv_scale must be 1-elem contiguous fp32 CUDA tensor");
     const at::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
-    auto q = torch::empty({x.numel() / 2}, torch::dtype(torch::kUInt8).device(x.device()));
+    auto q = new_tensor({x.numel() / 2}, torch::kUInt8, x);
     check_status(wush_quant_int4_tensor_scale(ptr<uint16_t>(x), ptr<uint8_t>(q), x.numel(), 0.0f,
                                               ptr<float>(inv_scale), current_stream(x)),
                  "quant_int4_tensor_scale_dev");
@@ -286,7 +306,7 @@ torch::Tensor gemm_tensor_scale_impl(torch::Tensor xq, torch::Tensor wq, double 
                 " (the per-tensor GEMM's int32 accumulator holds 256 * sum(qx * qw))");
     const int64_t N = wq.size(0);
     const at::hip::OptionalHIPGuardMasqueradingAsCUDA guard(xq.device());
-    auto y = torch::empty({M, N}, torch::dtype(torch::kHalf).device(xq.device()));
+    auto y = new_tensor({M, N}, torch::kHalf, xq);
     check_status(wush_gemm_s4_tensor_scale(ptr<uint8_t>(xq), ptr<uint8_t>(wq), ptr<uint16_t>(y), M, N,
                                            2 * K2, (float)alpha,
                                            alpha_dev ? ptr<float>(*alpha_dev) : nullptr, current_stream(xq)),
