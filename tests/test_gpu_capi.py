@@ -1160,6 +1160,33 @@ def test_per_tensor_quant_and_gemm(capi):
         assert np.array_equal(f16_tensor_f64(y), f16_tensor_f64(y2))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 33, 256), (127, 129, 256), (128, 256, 512), (129, 1001, 768), (300, 2050, 1024),
+                                   (700, 3001, 768), (1025, 4100, 1280), (260, 24580, 512), (4000, 4104, 256),
+                                   (9, 65536, 256)])
+def test_per_tensor_tiles_exact(capi, M, N, K):
+    # per-tensor tiles (K % 256 == 0) of every size and their edges, the
+    # 2-, 4- and 16-byte stores, one super-stage of K and more; codes over all
+    # of [-8, 7].  The int32 sum is exact and rounded once to fp16, so outputs
+    # equal fp16(fp32(dot) * alpha) bit for bit, for aligned and unaligned y.
+    import torch
+    g = rng(6200 + M + N)
+    xq, wq = pack_codes(g.integers(-8, 8, (M, K))), pack_codes(g.integers(-8, 8, (N, K)))
+    alpha = np.float32(1.0 / 48)
+    dx, dw = to_dev_u8(xq), to_dev_u8(wq)
+    rows, cols = _sample(g, M, 60), _sample(g, N, 1000)
+    dot = unpack_codes(xq[rows]).astype(np.int64) @ unpack_codes(wq[cols]).astype(np.int64).T
+    # alpha is scaled by 2^-8 in the kernel and the dot by 2^8: exact powers of two
+    exact = (dot.astype(np.float32) * alpha).astype(np.float16).astype(np.float64)
+    for off in (0, 1):
+        buf = torch.full((M * N + 16,), 7.0, dtype=torch.float16, device="cuda")
+        capi.gemm_s4_tensor_scale(dx.data_ptr(), dw.data_ptr(), buf.data_ptr() + 2 * off, M, N, K, float(alpha), None,
+                                  _stream())
+        torch.cuda.synchronize()
+        assert (buf[:off] == 7.0).all() and (buf[off + M * N:] == 7.0).all()
+        y = f16_tensor_f64(buf[off:off + M * N]).reshape(M, N)
+        assert np.array_equal(y[np.ix_(rows, cols)], exact), (M, N, K, off)
+
+
 def test_per_tensor_largest_k(capi):
     """K = 131040, the largest K the per-tensor GEMM admits (256 * 64 * K < 2^31):
     codes of -8 in both operands put every int32 accumulator at its extreme,

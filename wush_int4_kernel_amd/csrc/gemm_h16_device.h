@@ -1,8 +1,10 @@
-// gemm_h16_device.h -- device helpers shared by the fp16-MFMA prefill
-// kernels (gemm_h16.hip, gemm_h16q.hip): the code x scale -> fp16 operand
+// gemm_h16_device.h -- device helpers shared by the fp16-MFMA prefill kernels
+// (gemm_h16.hip, gemm_h16q.hip; gemm_pt.hip takes the tile order and loops): the code x scale -> fp16 operand
 // conversion, the MFMA fragment layout in LDS, the LDS DMA and the tile order.
 // See gemm_h16.hip for the numerics.
 #pragma once
+
+#include <utility>
 
 #include "wush_device.h"
 
@@ -164,6 +166,64 @@ __device__ __forceinline__ float h16_batch_scale(const uint32_t (&v)[kH16Batch],
     return __uint_as_float(v[i] << 16);
 }
 
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+
+// f(0), f(1), ..., f(N - 1) with compile-time arguments
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// c += a * b, accumulator in place.  The compiler does not know this is an
+// MFMA: the callers keep two instructions between a VALU write of an operand
+// and its use, and wait before reading c.
+__device__ __forceinline__ void mfma16_inplace(v4f& c, const h8& a, const h8& b) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+constexpr int kH16GroupRows = 8;                // row tiles walked together (tile order)
+
+// Tile index s in walking order -> (row tile, column tile): groups of
+// kH16GroupRows row tiles, all column tiles of a group before the next.
+// Workgroup i runs on XCD i % 8; each XCD takes a contiguous run of the
+// order, so the 32 workgroups in flight on it share 8 row tiles and a few
+// column tiles in its L2, for any tile counts.
+__device__ __forceinline__ void h16_tile(int id, int NR, int NC, int& tm, int& tn) {
+    const int total = NR * NC;
+    const int q = total >> 3, r = total & 7, x = id & 7;
+    const int s = x * q + min(x, r) + (id >> 3);
+    const int g = s / (kH16GroupRows * NC);
+    const int h = min(kH16GroupRows, NR - g * kH16GroupRows);
+    const int w = s - g * (kH16GroupRows * NC);
+    tm = g * kH16GroupRows + w % h;
+    tn = w / h;
+}
+
+// A wavefront's outputs, staged in LDS as `rows` rows of ROW bytes with
+// 16-byte chunk c of row r at chunk c ^ (r % (ROW / 16)), to y(m0.., n0..) one T
+// (uint16_t, or uint32_t for even N and 4-byte aligned y) per lane, so that an
+// instruction's stores are contiguous runs of a row: for the N that do not
+// allow 16-byte stores (700 x 3001 x 768 per-tensor product: 9.9 us, with
+// two-byte stores of 8 columns per lane, 16 bytes apart, 10.8).
+template <int ROW, typename T>
+__device__ __forceinline__ void store_staged(const uint8_t* stg, int rows, uint16_t* __restrict__ y, int m0, int M,
+                                             int n0, int N, int lane) {
+    constexpr int E = ROW / (int)sizeof(T), W = (int)sizeof(T) / 2;
+#pragma unroll 8
+    for (int k = 0; k < rows * E / 64; ++k) {
+        const int idx = k * 64 + lane;
+        const int r = idx / E, c = idx % E;      // element c of row r: columns W c ..
+        const int chunk = ((c * (int)sizeof(T)) >> 4) ^ (r & (ROW / 16 - 1));
+        const T v = *reinterpret_cast<const T*>(stg + r * ROW + chunk * 16 + ((c * (int)sizeof(T)) & 15));
+        if (m0 + r < M && n0 + W * c < N) *reinterpret_cast<T*>(y + (size_t)(m0 + r) * N + n0 + W * c) = v;
+    }
+}
 
 }  // namespace
 }  // namespace wush

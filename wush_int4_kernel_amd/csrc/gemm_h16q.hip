@@ -52,8 +52,6 @@
 // a library fp16 GEMM of the shape 2560-2850), M=256 238 -> 197, M=128 146 ->
 // 126; K=N=8192 M=4096 511 -> 431, M=512 116 -> 94; K=4096 N=24576 M=1024
 // 232 -> 185.
-#include <utility>
-
 #include "gemm_h16_device.h"
 #include "gemm_h16.h"
 #include "setup.h"
@@ -61,46 +59,7 @@
 namespace wush {
 namespace {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-
-// f(0), f(1), ..., f(N - 1) with compile-time arguments
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
-// c += a * b, accumulator in place.  The compiler does not know this is an
-// MFMA: the callers keep two instructions between a VALU write of an operand
-// and its use, and wait before reading c.
-__device__ __forceinline__ void mfma16_inplace(v4f& c, const h8& a, const h8& b) {
-    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-
 constexpr int kH16qStage = kH16Tile * 64;        // workspace bytes of one stage of a 256-row tile
-constexpr int kH16qGroupRows = 8;                // row tiles walked together (tile order)
-
-// Tile index s in walking order -> (row tile, column tile): groups of
-// kH16qGroupRows row tiles, all column tiles of a group before the next.
-// Workgroup i runs on XCD i % 8; each XCD takes a contiguous run of the
-// order, so the 32 workgroups in flight on it share 8 row tiles and a few
-// column tiles in its L2, for any tile counts.
-__device__ __forceinline__ void h16q_tile(int id, int NR, int NC, int& tm, int& tn) {
-    const int total = NR * NC;
-    const int q = total >> 3, r = total & 7, x = id & 7;
-    const int s = x * q + min(x, r) + (id >> 3);
-    const int g = s / (kH16qGroupRows * NC);
-    const int h = min(kH16qGroupRows, NR - g * kH16qGroupRows);
-    const int w = s - g * (kH16qGroupRows * NC);
-    tm = g * kH16qGroupRows + w % h;
-    tn = w / h;
-}
-
 // RB: 16-row blocks per wavefront, 16 (256-row tiles) or 8 (128-row tiles:
 // half the accumulators, the same weight conversion per stage).
 template <int RB>
@@ -129,7 +88,7 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
     const int mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile, npad = NC * kH16Tile;
     const int slice = blockIdx.x / (NR * NC);
     int tm, tn;
-    h16q_tile((int)blockIdx.x - slice * (NR * NC), NR, NC, tm, tn);
+    h16_tile((int)blockIdx.x - slice * (NR * NC), NR, NC, tm, tn);
     const int m0 = tm * TR;
     const int n0 = tn * TC;
     const int gb = slice * groups_per_split;

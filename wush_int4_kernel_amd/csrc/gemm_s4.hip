@@ -28,6 +28,7 @@
 
 #include "wush_device.h"
 #include "gemm_h16.h"
+#include "gemm_pt.h"
 #include "setup.h"
 #include "../../include/wush_int4.h"
 
@@ -979,6 +980,35 @@ static size_t best_bytes(int64_t M, int64_t N, int64_t K, size_t base) {
     return p.a16 && N < WUSH_H16A_MIN_N ? std::max(b, base + 256) : base;
 }
 
+// Per-tensor route: the tiles of gemm_pt.hip for K % 256 == 0, unless a few
+// activation rows (M <= 32) would fill only the corner of more than one round
+// of 128 x 128 tiles (M = 1, 448 tiles of K=8192: 61 us against 50 with the
+// 32-row int8 tiles; 192 tiles at M = 8 16.3 against 19.6).
+// The tile is the cheapest by an estimate in us, per round of up to 256
+// workgroups: a fixed cost, and per 256 codes of K a cost that grows with the
+// workgroups running (the clock follows the power).  Measured on MI355X: 2048
+// x 4096 x 4096 43.3 / 30.7 / 34.0 us with 256x256 / 256x128 / 128x128 tiles,
+// 4096^3 52 / 60 / 68, 512 x 24576 x 4096 46.6 / 53.7 / 49.6, 1000 x 4096 x
+// 12288 105 / 66 / 44, 256 x 4096 x 4096 40 / 25.5 / 16.2.
+static bool plan_pt(int64_t M, int64_t N, int64_t K, int* rows, int* cols) {
+    if (K % 256 != 0 || (M <= 32 && N > 32768)) return false;
+    static const struct { int rows, cols; double fixed, lo, hi; } kTiles[] = {
+        {256, 256, 7.0, 1.94, 2.70}, {256, 128, 4.0, 1.24, 1.60}, {128, 128, 2.0, 0.79, 0.92}};
+    double best = 0.0;
+    for (const auto& t : kTiles) {
+        const int64_t wgs = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
+        const double steps = (double)(K / 256);
+        auto round_us = [&](int64_t n) { return n ? t.fixed + steps * (t.lo + (t.hi - t.lo) * (double)n / 256.0) : 0.0; };
+        const double us = (double)(wgs / 256) * round_us(256) + round_us(wgs % 256);
+        if (best == 0.0 || us < best) {
+            best = us;
+            *rows = t.rows;
+            *cols = t.cols;
+        }
+    }
+    return true;
+}
+
 template <int BM, int BN, int WM, int WN, int SG, int MR, bool PT>
 static void launch_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
                         uint16_t* y, float* partial, int M, int N, int K, const Plan& p, float alpha,
@@ -1018,6 +1048,11 @@ static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, co
                             reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
     // the pre-converted activations need a 16-byte aligned workspace
     allow_a16 = allow_a16 && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
+    if constexpr (PT) {
+        int rows = 0, cols = 0;
+        if (plan_pt(M, N, K, &rows, &cols))
+            return launch_gemm_pt(xq, wq, y, (int)M, (int)N, (int)K, alpha, alpha_dev, rows, cols, stream);
+    }
     const size_t room = workspace ? ws_bytes : 0;
     bool narrow_a16 = false;
     if (!PT && allow_a16 && N < WUSH_H16A_MIN_N && room > 0 && h16a_preferred(M, N, K))
