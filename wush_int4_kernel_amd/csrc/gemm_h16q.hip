@@ -312,24 +312,22 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
         __builtin_amdgcn_sched_barrier(0);       // one column block at a time
     }
     const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-    const int r0 = lane >> 3, cc = lane & 7;
-    const int n = wn0 + cc * 8;
-    const uint8_t* rst = stg + r0 * 128 + (cc ^ r0) * 16;    // row 8 k + r0: (8 k + r0) % 8 == r0
-    uint16_t* yrow = y + (size_t)(m0 + r0) * N + n;
+    // the lane number again: kept from the start it would spill a register
+    const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    if (vec) {
+        const int r0 = ln >> 3, cc = ln & 7;
+        const int n = wn0 + cc * 8;
+        const uint8_t* rst = stg + r0 * 128 + (cc ^ r0) * 16;    // row 8 k + r0: (8 k + r0) % 8 == r0
+        uint16_t* yrow = y + (size_t)(m0 + r0) * N + n;
 #pragma unroll
-    for (int k = 0; k < TR / 8; ++k) {
-        const uint4 v = *reinterpret_cast<const uint4*>(rst + k * 1024);
-        if (m0 + 8 * k + r0 < M) {
-            uint16_t* dst = yrow + (size_t)(8 * k) * N;
-            if (vec) {
-                if (n < N) *reinterpret_cast<uint4*>(dst) = v;
-            } else {
-                const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (n + e < N) dst[e] = (uint16_t)(d[e >> 1] >> (16 * (e & 1)));
-            }
+        for (int k = 0; k < TR / 8; ++k) {
+            const uint4 v = *reinterpret_cast<const uint4*>(rst + k * 1024);
+            if (m0 + 8 * k + r0 < M && n < N) *reinterpret_cast<uint4*>(yrow + (size_t)(8 * k) * N) = v;
         }
+    } else if ((N & 1) == 0 && (reinterpret_cast<uintptr_t>(y) & 3u) == 0) {
+        store_staged<128, uint32_t>(stg, TR, y, m0, M, wn0, N, ln);
+    } else {
+        store_staged<128, uint16_t>(stg, TR, y, m0, M, wn0, N, ln);
     }
     if (bad != 0) {
         WUSH_WAIT_VMCNT(0);
