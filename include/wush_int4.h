@@ -109,14 +109,14 @@ int wush_gemv_int4_supported(int64_t M, int64_t N, int64_t K);
 /* Bytes of workspace wush_gemm_s4 uses for (M, N, K); 0 when it needs none:
  * fp32 split-K partials, and for prefill shapes with N >= 8192 the
  * activations converted once to fp16 operands (M*K*2 bytes, padded to 256
- * rows).  A caller may pass a larger buffer; a smaller one makes wush_gemm_s4
+ * rows and 256 of K).  A caller may pass a larger buffer; a smaller one makes wush_gemm_s4
  * choose a plan that needs no more than it is given (same results). */
 size_t wush_gemm_s4_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* Bytes of workspace with which wush_gemm_s4 runs its fastest plan; at least
  * wush_gemm_s4_workspace_bytes, and more where that plan also converts the
  * activations to fp16 operands on weights of fewer than 8192 rows (M > 64,
- * K % 256 == 0, 16-byte aligned scales, from about 2^32 multiply-adds): with
+ * K % 64 == 0, 16-byte aligned scales, from about 2^32 multiply-adds): with
  * fewer bytes than this, wush_gemm_s4 runs the plan of
  * wush_gemm_s4_workspace_bytes there.  The reference has no counterpart. */
 size_t wush_gemm_s4_best_workspace_bytes(int64_t M, int64_t N, int64_t K);
@@ -125,9 +125,9 @@ size_t wush_gemm_s4_best_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * wush_gemv_int4, y (M, N) fp16.  On int8 MFMA with exact int32 group dots,
  * except for three ranges that run fp16 MFMA on code*scale operands (exact
  * after a power-of-two shift per row and column) accumulated in fp32 over all
- * of K: M > 64 with K % 256 == 0, from about 2^32 multiply-adds (3e9; 4.8e9 for
- * N < 2048; 192 tiles of 128 x 256 outputs at N >= 8192), when the workspace
- * holds the converted activations (see the two functions above); without that
+ * of K: M > 64 with K % 64 == 0, from about 2^32 multiply-adds (3e9, 4.8e9 for
+ * N < 2048; twice that for K % 256 != 0; or 192 tiles of 128 x 256 outputs at
+ * N >= 8192 and K % 256 == 0), when the workspace holds the converted activations (see the two functions above); without that
  * room M > 128 with K % 256 == 0, at least 64 tiles of 256x256 or N >= 2048, and
  * at least 128 workgroups counting the K slices of at least 32 groups each
  * that the workspace holds from M = 512; and 32 < M <= 64 with 49953 <= N <=

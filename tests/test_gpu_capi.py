@@ -937,7 +937,9 @@ def test_gemm_h16_nonfinite_scales(capi, M, N):
                                    (130, 8196, 6144),     # ... 16-byte partial stores, fp16 rows of 8 bytes
                                    (129, 33001, 256),     # one double batch, scalar fp16 stores
                                    (257, 32772, 768),     # a one-row second tile, 8-byte rows
-                                   (65, 49155, 512)])     # scalar fp16 stores
+                                   (65, 49155, 512),      # scalar fp16 stores
+                                   (203, 8195, 8256),     # K % 256 == 64: last 8-group block of 2, K split unevenly
+                                   (130, 16390, 4288)])   # ... of 6
 def test_gemm_h16q_ragged_columns(capi, M, N, K):
     # converted-activation tiles whose rows of y are not whole 16-byte chunks,
     # with a non-finite row and a non-finite last column (split plans write
@@ -959,10 +961,12 @@ def test_gemm_h16q_ragged_columns(capi, M, N, K):
 
 
 # Narrow weights (N < 8192): every tile height (64, 128, 256 rows) and K splits
-# from 1 to 16, ragged M and N, G = K / 32 that splits by 8 only once
+# from 1 to 16, ragged M and N, K that is a multiple of 64 only (the last
+# block of 8 groups holds 2, 4 or 6), splits of unequal length
 @pytest.mark.parametrize("M,N,K", [(65, 4096, 16384), (256, 4096, 4096), (512, 4099, 4096), (129, 6146, 6144),
                                    (1000, 2051, 2304), (1030, 4096, 2048), (2047, 4100, 2048), (4090, 4104, 512),
-                                   (400, 1027, 14336), (70, 8190, 8192)])
+                                   (400, 1027, 14336), (70, 8190, 8192), (700, 4099, 2240), (3000, 2050, 1088),
+                                   (256, 4100, 8384), (5000, 4104, 320), (70, 7000, 12352)])
 def test_gemm_best_workspace_plan_agrees(capi, M, N, K):
     # the converted-activation plan, taken from
     # wush_gemm_s4_best_workspace_bytes on, and the plan of the bytes that

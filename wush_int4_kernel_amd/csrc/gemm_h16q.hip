@@ -61,8 +61,12 @@ namespace {
 
 constexpr int kH16qStage = kH16Tile * 64;        // workspace bytes of one stage of a 256-row tile
 // RB: 16-row blocks per wavefront, 16 (256-row tiles) or 8 (128-row tiles:
-// half the accumulators, the same weight conversion per stage).
-template <int RB>
+// half the accumulators, the same weight conversion per stage) or 4.  PAD: K is
+// a multiple of 64 but not of 256: the last double batch reads the row's last
+// groups again in place of those past the end, whose activations and weight
+// scales are zero, and scales come 4 bytes at a time (rows of them are only
+// 4-byte aligned).
+template <int RB, bool PAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ ea, const int* __restrict__ eb,
                       const uint8_t* __restrict__ wq, const uint16_t* __restrict__ ws, uint16_t* __restrict__ y,
@@ -81,7 +85,7 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
     const int l16 = lane & 15, kq = lane >> 4;   // row or column of an operand, lane quarter
-    const int GR = K >> 5;
+    const int GR = K >> 5, GP = PAD ? (GR + 7) & ~7 : GR;   // groups of a row, and whole double batches of them
     const int K2 = K >> 1;
     const int NR = (M + TR - 1) / TR, NC = (N + TC - 1) / TC;
     // shifts and converted activations are laid out over 256-row padding
@@ -92,11 +96,11 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
     const int m0 = tm * TR;
     const int n0 = tn * TC;
     const int gb = slice * groups_per_split;
-    const int G = min(GR - gb, groups_per_split);
+    const int G = min(GP - gb, groups_per_split);
     const uint32_t lds0 = lds_addr(smem);
 
     // activation DMA of this wavefront: KiB NA w .. NA w + NA - 1 of a stage
-    const uint8_t* asrc = a16 + ((size_t)(m0 >> 8) * GR + gb) * kH16qStage + (m0 & 255) * 64 + wave * (NA * 1024);
+    const uint8_t* asrc = a16 + ((size_t)(m0 >> 8) * GP + gb) * kH16qStage + (m0 & 255) * 64 + wave * (NA * 1024);
     const uint32_t avoff = lane * 16;
     auto issue_a = [&](int st, int slot, int d) {    // past the slice: the last stage
         dma16_uniform(asrc + (size_t)min(st, G - 1) * kH16qStage + d * 1024, avoff,
@@ -113,12 +117,22 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
         const int c = 8 * k + (lane >> 3);
         const int p = (lane & 7) ^ ((c >> 1) & 7);
         const int col = min(col0 + c, N - 1);
-        dma16(wq + (size_t)col * K2 + (size_t)(gb + o) * 16 + p * 16,
+        const int g = PAD ? min(gb + o + p, GR - 1) : gb + o + p;
+        dma16(wq + (size_t)col * K2 + (size_t)g * 16,
               lds0 + kCodes + (buf * 4 + wave) * 8192 + k * 1024);
     };
-    const uint16_t* ssrc = ws + (size_t)min(col0 + lane, N - 1) * GR + gb;
+    // scales of a double batch: [column][8 groups], PAD: [group pair][column][2]
+    constexpr int kScaleDmas = PAD ? 4 : 1;
+    const uint16_t* ssrc = ws + (size_t)min(col0 + lane, N - 1) * GR;
     auto issue_s = [&](int d, int buf) {
-        dma16(ssrc + min(d * 8, G - 8), lds0 + kScales + (buf * 4 + wave) * 1024);
+        const int g = gb + min(d * 8, G - 8);
+        const uint32_t dst = lds0 + kScales + (buf * 4 + wave) * 1024;
+        if constexpr (PAD) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) dma4(ssrc + min(g + 2 * k, GR - 2), dst + k * 256);
+        } else {
+            dma16(ssrc + g, dst);
+        }
     };
 
     v4f acc[RB][4];
@@ -141,11 +155,19 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
     auto read_batch = [&](int b, Batch& r) {
         const uint8_t* cb = smem + kCodes + (((b >> 1) & 1) * 4 + wave) * 8192 + l16 * 128 +
                             16 * ((4 * (b & 1) + kq) ^ fsw);
-        const uint8_t* sb = smem + kScales + (((b >> 1) & 1) * 4 + wave) * 1024 + l16 * 16 + 2 * (4 * (b & 1) + kq);
+        const int gq = 4 * (b & 1) + kq;         // the lane's group of the double batch
+        const uint8_t* sb = smem + kScales + (((b >> 1) & 1) * 4 + wave) * 1024 +
+                            (PAD ? (gq >> 1) * 256 + l16 * 4 + 2 * (gq & 1) : l16 * 16 + 2 * gq);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             r.c[j] = *reinterpret_cast<const u32v4*>(cb + j * 2048);
-            sraw[j] = *reinterpret_cast<const uint16_t*>(sb + j * 256);
+            sraw[j] = *reinterpret_cast<const uint16_t*>(sb + j * (PAD ? 64 : 256));
+        }
+        if constexpr (PAD) {
+            if (gb + 4 * b + kq >= GR) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sraw[j] = 0;
+            }
         }
     };
     auto make_scale = [&](Batch& r, int j) { r.s[j] = h16_scale(__uint_as_float(sraw[j] << 16), ecol[j]); };
@@ -198,6 +220,7 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
     static_for<52>([&](auto k) { convert_step(0, R[0], 0, k.value); });
 #pragma unroll
     for (int i = 0; i < RB; ++i) read_a(0, 0, i);
+    asm volatile("s_nop 7");                     // the zeroed accumulators before the first MFMA
     __builtin_amdgcn_sched_barrier(0);
 
     for (int s0 = 0; s0 < G; s0 += 8) {
@@ -237,7 +260,7 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
                 static_for<k1 - k0>([&](auto k) { convert_step(P ^ 1, Rc, (j + 1) & 3, k0 + k.value); });
                 __builtin_amdgcn_sched_barrier(0);
             });
-            if constexpr (j == 4 || j == 5) WUSH_WAIT_VMCNT(kInFlight + 1);   // the scale DMA of j = 4
+            if constexpr (j == 4 || j == 5) WUSH_WAIT_VMCNT(kInFlight + kScaleDmas);   // the scales of j = 4
             else WUSH_WAIT_VMCNT(kInFlight);
             WUSH_LDS_BARRIER();
             __builtin_amdgcn_sched_barrier(0);
@@ -354,8 +377,16 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
 // HBM-bound: 4096 x 8192 in 17.4 us (4.9 TB/s over 84 MB), against 28.5 us
 // with each thread loading 16 bytes of its own row and one 32-row block per
 // workgroup (most of a wave of workgroups idle at small M).
+// PAD: G % 8 != 0, so rows of scales are 4-byte aligned (G is even).
+template <bool PAD>
 __device__ __forceinline__ uint32_t slice_scale_max(const uint16_t* p, int n, int part) {
     u16x2 m2 = {0, 0};
+    if constexpr (PAD) {
+        const uint32_t* p1 = reinterpret_cast<const uint32_t*>(p);
+#pragma unroll 4
+        for (int i = part; i < (n >> 1); i += 8) m2 = __builtin_elementwise_max(m2, abs_bits2(p1[i]));
+        return max((uint32_t)m2.x, (uint32_t)m2.y);
+    }
     const uint4* p4 = reinterpret_cast<const uint4*>(p);
 #pragma unroll 4
     for (int i = part; i < (n >> 3); i += 8) {
@@ -368,6 +399,7 @@ __device__ __forceinline__ uint32_t slice_scale_max(const uint16_t* p, int n, in
 
 constexpr int kPrepChunk = 32;                   // groups per converting workgroup
 
+template <bool PAD>
 __global__ __launch_bounds__(256) void h16_prep_kernel(const uint8_t* __restrict__ xq,
                                                        const uint16_t* __restrict__ xs,
                                                        uint8_t* __restrict__ a16, int* __restrict__ ea,
@@ -385,7 +417,7 @@ __global__ __launch_bounds__(256) void h16_prep_kernel(const uint8_t* __restrict
     const int sg0 = slice * groups_per_split, sg1 = min(G, sg0 + groups_per_split);
     const int row = blk * 32 + r;
     const bool ok = row < (wside ? N : M);
-    uint32_t mx = ok ? slice_scale_max((wside ? ws : xs) + (size_t)row * G + sg0, sg1 - sg0, part) : 0x3f80u;
+    uint32_t mx = ok ? slice_scale_max<PAD>((wside ? ws : xs) + (size_t)row * G + sg0, sg1 - sg0, part) : 0x3f80u;
     mx = max(mx, (uint32_t)__shfl_xor((int)mx, 1));
     mx = max(mx, (uint32_t)__shfl_xor((int)mx, 2));
     mx = max(mx, (uint32_t)__shfl_xor((int)mx, 4));
@@ -397,13 +429,14 @@ __global__ __launch_bounds__(256) void h16_prep_kernel(const uint8_t* __restrict
     if (part == 0 && chunk == 0) ea[(size_t)slice * (mblocks * 32) + row] = !ok || e == kH16NonFinite ? 0 : -e;
     const uint8_t* q = xq + (size_t)row * G * 16;
     const uint16_t* s = xs + (size_t)row * G;
-    uint8_t* dst = a16 + (size_t)(blk >> 3) * G * kH16qStage + (blk & 7) * 2048 + (r >> 4) * 1024 + (r & 15) * 16;
-    const int g1 = min(sg1, sg0 + (chunk + 1) * kPrepChunk);
+    const int GP = PAD ? (G + 7) & ~7 : G;
+    uint8_t* dst = a16 + (size_t)(blk >> 3) * GP * kH16qStage + (blk & 7) * 2048 + (r >> 4) * 1024 + (r & 15) * 16;
+    const int g1 = min(min(GP, sg0 + groups_per_split), sg0 + (chunk + 1) * kPrepChunk);
 #pragma unroll 4
     for (int g = sg0 + chunk * kPrepChunk + part; g < g1; g += 8) {
         uint4 w = {0, 0, 0, 0};
         float f = 0.0f;
-        if (ok) {
+        if (ok && (!PAD || g < G)) {
             w = *reinterpret_cast<const uint4*>(q + (size_t)g * 16);
             f = __uint_as_float((uint32_t)s[g] << 16);
         }
@@ -422,14 +455,14 @@ __global__ __launch_bounds__(256) void h16_prep_kernel(const uint8_t* __restrict
 size_t gemm_h16a_workspace_bytes(int64_t M, int64_t N, int64_t K, int splits) {
     const int64_t mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile;
     const int64_t npad = (N + kH16Tile - 1) / kH16Tile * kH16Tile;
-    return (size_t)mpad * (size_t)K * 2 + (size_t)splits * (size_t)(mpad + npad) * sizeof(int);
+    return (size_t)mpad * (size_t)((K + 255) / 256 * 256) * 2 + (size_t)splits * (size_t)(mpad + npad) * sizeof(int);
 }
 
 int launch_gemm_h16a(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
                      uint16_t* y, float* partial, int M, int N, int K, int splits, int groups_per_split,
                      void* a_ws, int tile_rows, hipStream_t stream) {
     const int G = K >> 5;
-    if (M <= 0 || N <= 0 || K <= 0 || K % 256 != 0 || splits < 1 || groups_per_split <= 0 ||
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || splits < 1 || groups_per_split <= 0 ||
         groups_per_split % 8 != 0 || (long long)splits * groups_per_split < G ||
         (tile_rows != 64 && tile_rows != 128 && tile_rows != 256) ||
         (long long)(splits - 1) * groups_per_split >= G || (splits > 1 && partial == nullptr) || a_ws == nullptr ||
@@ -439,18 +472,22 @@ int launch_gemm_h16a(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, c
     const int mpad = (M + kH16Tile - 1) / kH16Tile * kH16Tile;
     const int npad = (N + kH16Tile - 1) / kH16Tile * kH16Tile;
     uint8_t* a16 = static_cast<uint8_t*>(a_ws);
-    int* ea = reinterpret_cast<int*>(a16 + (size_t)mpad * K * 2);
+    const bool pad = G % 8 != 0;
+    int* ea = reinterpret_cast<int*>(a16 + (size_t)mpad * ((K + 255) / 256 * 256) * 2);
     int* eb = ea + (size_t)splits * mpad;
     const int mblocks = mpad / 32, nblocks = npad / 32;
     const int chunks = (groups_per_split + kPrepChunk - 1) / kPrepChunk;
     const long long na = (long long)mblocks * splits * chunks, nprep = na + (long long)nblocks * splits;
     const long long tiles = (long long)((N + kH16Tile - 1) / kH16Tile) * ((M + tile_rows - 1) / tile_rows) * splits;
     if (nprep > 0x7fffffffLL || tiles > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-    h16_prep_kernel<<<dim3((unsigned)nprep), 256, 0, stream>>>(xq, xs, a16, ea, ws, eb, M, N, G, groups_per_split,
-                                                               mblocks, nblocks, chunks, (int)na);
+    const auto prep = pad ? h16_prep_kernel<true> : h16_prep_kernel<false>;
+    prep<<<dim3((unsigned)nprep), 256, 0, stream>>>(xq, xs, a16, ea, ws, eb, M, N, G, groups_per_split, mblocks, nblocks,
+                                                    chunks, (int)na);
     const int e = (int)hipGetLastError();
     if (e != 0) return e;
-    const auto kernel = tile_rows == 64 ? gemm_h16q_kernel<4> : tile_rows == 128 ? gemm_h16q_kernel<8> : gemm_h16q_kernel<16>;
+    const auto kernel = tile_rows == 64    ? (pad ? gemm_h16q_kernel<4, true> : gemm_h16q_kernel<4, false>)
+                        : tile_rows == 128 ? (pad ? gemm_h16q_kernel<8, true> : gemm_h16q_kernel<8, false>)
+                                           : (pad ? gemm_h16q_kernel<16, true> : gemm_h16q_kernel<16, false>);
     kernel<<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K, groups_per_split);
     return (int)hipGetLastError();
 }

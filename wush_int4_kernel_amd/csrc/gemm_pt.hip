@@ -117,6 +117,7 @@ void gemm_pt_kernel(const uint8_t* __restrict__ xq, const uint8_t* __restrict__ 
         for (int j = 0; j < CB; ++j) unpack(ub[0][j], rb[0][j], 0, t);
         unpack(ua[0], ra[0][0], 0, t);
     }
+    asm volatile("s_nop 7");                     // the zeroed accumulators before the first MFMA
     __builtin_amdgcn_sched_barrier(0);
 
     int buf = 0;                                 // LDS buffer of super-stage st

@@ -758,7 +758,7 @@ static size_t plan_bytes(const Plan& p, int64_t M, int64_t N, int64_t K) {
 #ifndef WUSH_H16_SPLIT_MIN_M
 #define WUSH_H16_SPLIT_MIN_M 512
 #endif
-// Converted-activation fp16 tiles (gemm_h16q.hip), M > 64, K % 256 == 0,
+// Converted-activation fp16 tiles (gemm_h16q.hip), M > 64, K % 64 == 0,
 // 16-byte aligned scales and room in the workspace.  They cost three launches
 // (conversion, GEMM, split-K sum) where the int8 tiles cost one or two, so
 // they take over from this many multiply-adds: M=N=4096-wide K=4096 at M=256
@@ -825,10 +825,15 @@ constexpr int kStream32Waves = WUSH_S32_WAVES;
 
 // Whether the converted-activation fp16 tiles run (M, N, K), given the room.
 static bool h16a_preferred(int64_t M, int64_t N, int64_t K) {
-    if (K % 256 != 0 || M <= 64) return false;
-    const double work = (double)M * (double)N * (double)K;
+    if (K % 64 != 0 || M <= 64) return false;
+    // a short last block of 8 groups costs a whole one: K = 1088 counts as
+    // 1280, and 2048 x 2048 x 1088 (1.06 of 2^32) took 33.0 us against 29.6 with
+    // the int8 tiles, so such K take twice the work (300 x 11008 x 2880, 2.2 of
+    // 2^32: 60.8 -> 47.1; 1000 x 4096 x 4160 82.7 -> 66.8)
+    const double work = (double)M * (double)N * (double)K / (K % 256 != 0 ? 2.0 : 1.0);
     if (work >= (N < WUSH_H16A_NARROW_N ? (double)WUSH_H16A_NARROW_MIN_WORK : (double)WUSH_H16A_MIN_WORK)) return true;
-    return N >= WUSH_H16A_MIN_N && ((M + 127) / 128) * ((N + 255) / 256) >= WUSH_H16A_MIN_TILES;
+    return K % 256 == 0 && N >= WUSH_H16A_MIN_N &&
+           ((M + 127) / 128) * ((N + 255) / 256) >= WUSH_H16A_MIN_TILES;
 }
 
 // Estimated us of the converted-activation tiles with `rows`-row tiles and s
@@ -840,12 +845,12 @@ static bool h16a_preferred(int64_t M, int64_t N, int64_t K) {
 // 512 <= N <= 65536, 256 <= K <= 16384, every tile height and K split): the
 // tile and split with the least estimate is on average 0.7% slower than the
 // best one measured, 10% at worst.
-static double h16a_cost_us(int64_t M, int64_t N, int64_t K, int rows, int s) {
+static double h16a_cost_us(int64_t M, int64_t N, int64_t K, int rows, int s, int groups_per_split) {
     static const struct { int rows; double fixed, lo, hi; } kCost[] = {
         {64, 3.5, 0.225, 0.275}, {128, 4.5, 0.3125, 0.40}, {256, 8.0, 0.50, 0.66}};
     const auto& c = kCost[rows == 64 ? 0 : rows == 128 ? 1 : 2];
     const int64_t wgs = ((M + rows - 1) / rows) * ((N + 255) / 256) * s;
-    const double stages = (double)(K / 32) / s;
+    const double stages = (double)groups_per_split;
     auto round_us = [&](int64_t n) { return n ? c.fixed + stages * (c.lo + (c.hi - c.lo) * (double)n / 256.0) : 0.0; };
     double us = 5.0 + (double)(wgs / 256) * round_us(256) + round_us(wgs % 256);
     us += (2.5 * (double)M * (double)K + (double)N * (double)K / 16.0) / 5e6;
@@ -856,19 +861,21 @@ static double h16a_cost_us(int64_t M, int64_t N, int64_t K, int rows, int s) {
 // The cheapest tile height and K split (slices of whole 8-group blocks) whose
 // workspace fits `room`; false if none does.
 static bool plan_h16a(int64_t M, int64_t N, int64_t K, size_t room, Plan* out) {
-    const int64_t G = K / 32;
+    const int64_t G = K / 32, blocks = (G + 7) / 8;   // the last 8-group block may be short
     double best = 0.0;
     bool found = false;
     for (int rows = 64; rows <= 256; rows *= 2) {
         if (rows > 64 && M <= rows / 2) break;
-        for (int s = 1; s <= 16 && G % (8 * s) == 0; s *= 2) {
+        for (int s = 1; s <= 16 && s <= blocks; s *= 2) {
+            const int64_t gps = (blocks + s - 1) / s * 8;
+            if ((s - 1) * gps >= G) continue;         // a slice would be empty
             Plan q;
             q.cfg = 5; q.mr = 32; q.tm = rows; q.tn = 256; q.sg = 1;
             q.splits = s;
-            q.groups_per_split = (int)(G / s);
+            q.groups_per_split = (int)gps;
             q.a16 = true;
             if (plan_bytes(q, M, N, K) > room) break;
-            const double us = h16a_cost_us(M, N, K, rows, s);
+            const double us = h16a_cost_us(M, N, K, rows, s, (int)gps);
             if (!found || us < best) { *out = q; best = us; found = true; }
         }
     }
