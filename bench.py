@@ -161,14 +161,14 @@ def ref_reps(M: int) -> int:
 
 
 def prefill_mfma(M: int, N: int, K: int) -> str:
-    """MFMA type of the w4a4_gemm_s4 kernel for M rows at the bench's shapes:
-    the fp16 tiles from M = 256 when K % 256 == 0 (every bench shape has at
-    least 16 column tiles of 256, which with M >= 256 meets the planner's
-    tile-count condition, except Qwen3-8B K=N=4096 below M = 2048), the fp16
-    streaming kernel at 32 < M <= 64 when 224 to 256 workgroups of 224
-    columns cover N and K % 1024 == 0, int8 otherwise."""
+    """MFMA type of the w4a4_gemm_s4 kernel for M rows at the bench's shapes
+    (N >= 512, K % 256 == 0): the fp16 tiles from M = 65 and 3e9 multiply-adds
+    (4.8e9 on fewer than 2048 columns), the fp16 streaming kernel at
+    32 < M <= 64 when 224 to 256 workgroups of 224 columns cover N and
+    K % 1024 == 0, int8 otherwise."""
     wgs = -(-N // 224)
-    if (M >= 256 and K % 256 == 0) or (32 < M <= 64 and 224 <= wgs <= 256 and K % 1024 == 0):
+    tiles = M > 64 and K % 256 == 0 and M * N * K >= (3e9 if N >= 2048 else 4.8e9)
+    if tiles or (32 < M <= 64 and 224 <= wgs <= 256 and K % 1024 == 0):
         return "fp16"
     return "int8"
 

@@ -158,7 +158,7 @@ int wush_gemm_s4(const uint8_t *xq, const uint16_t *xs, const uint8_t *wq, const
  * bit: a shape whose full split of K would need more partials than the
  * scratch holds is split into fewer slices.  The scratch never holds
  * converted activations, so where wush_gemm_s4 with a workspace converts them
- * once (N >= 8192 at M > 64, on enough workgroups) this entry point runs the
+ * once (M > 64, from about 2^32 multiply-adds) this entry point runs the
  * per-tile fp16 tiles or the int8 tiles: equal to the parity tolerance, not
  * bit for bit.  Nothing needs clearing
  * between calls: every partial is written before it is summed.  All calls on

@@ -351,7 +351,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("alpha"));
     m.def("w4a4_gemm_s4", &w4a4_gemm_s4,
           "W4A4 group-scaled matmul: int8 MFMA with exact int32 group dots below prefill sizes, fp16 MFMA on "
-          "code*scale operands for prefill (M >= 256)",
+          "code*scale operands for prefill (M > 64)",
           py::arg("xq"),
           py::arg("xs"), py::arg("wq"), py::arg("ws"));
     m.def("s4_atom_selftest", &s4_atom_selftest, "verify the int8 MFMA fragment layout");

@@ -683,7 +683,7 @@ __global__ void mfma_selftest_kernel(const int8_t* __restrict__ a, const int8_t*
 struct Plan {
     int cfg;        // 0: 32x128 (M <= 32), 1: 64x128, 2: 128x128,
                     // 4: streaming with in-workgroup K split (M <= 64),
-                    // 5: 256x256 fp16-MFMA tiles (gemm_h16.hip),
+                    // 5: fp16-MFMA tiles (a16: gemm_h16q.hip, tm rows; else gemm_h16.hip, 256x256),
                     // 6: fp16-MFMA streaming, 8 < M <= 64 (gemm_h16s.hip)
     int mr;         // fold rows per 32-row block (cfg 0, 4)
     int splits;
@@ -714,7 +714,8 @@ static size_t plan_bytes(const Plan& p, int64_t M, int64_t N, int64_t K) {
 #ifndef WUSH_PF_BN
 #define WUSH_PF_BN 2             // and along N (2 x 2 wavefronts per workgroup)
 #endif
-// fp16-MFMA 256x256 tiles (gemm_h16.hip) from this M when they make at least
+// Per-tile fp16-MFMA 256x256 tiles (gemm_h16.hip; where the workspace has no room
+// for converted activations) from this M when they make at least
 // this many tiles (K % 256 == 0).  Against the int8 tiles on MI355X: L70
 // M=256 (224 tiles) 249 vs 392 us, M=2048 K=N=4096 (128) 108 vs 128,
 // M=1024 K=N=8192 (128) 195 vs 217; L70 M=160 251 vs 434, M=192 239 vs 410,
