@@ -62,6 +62,45 @@ def test_library_exports_no_undeclared_c_symbols():
     assert exported == declared_symbols()
 
 
+def test_lds_dma_waits_for_its_m0_write(tmp_path):
+    # gfx950 needs one wait state between a scalar write of M0 and the LDS DMA
+    # that takes its LDS address from M0.  The compiler inserts it for its own
+    # instructions, not inside the asm strings of wush_device.h, so the built
+    # code is checked: no DMA directly behind a write of M0.  Nor does it see
+    # that such an asm reads an SGPR as a vector memory address, which needs
+    # five wait states after a VALU write of that SGPR.
+    import glob
+    import shutil
+    import subprocess
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    lib = shutil.copy(os.path.join(ROOT, "wush_int4_kernel_amd", "libwush_int4.so"), tmp_path)
+    subprocess.run([objdump, "--offloading", lib], cwd=tmp_path, capture_output=True, check=True)
+    dmas, early = 0, []
+    for obj in sorted(glob.glob(str(tmp_path / "*gfx950"))):
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", obj], capture_output=True, text=True,
+                              check=True).stdout
+        ins = [line.split("//")[0].strip() for line in text.splitlines() if line.startswith("\t")]
+        for i, op in enumerate(ins):
+            if not re.match(r"(global|buffer|flat|scratch)_", op):
+                continue
+            if re.match(r"global_load_lds_|buffer_load_\w+ .*\blds\b", op):
+                dmas += 1
+                if re.match(r"s_\w+ m0,", ins[i - 1]):
+                    early.append((ins[i - 1], op))
+            sgprs = {r for a, b in re.findall(r"\bs\[(\d+):(\d+)\]", op) for r in range(int(a), int(b) + 1)}
+            waited = 0
+            for prev in reversed(ins[max(0, i - 5):i]):
+                wrote = re.match(r"v_\w+ s(?:(\d+)|\[(\d+):(\d+)\]),", prev)
+                if wrote and waited < 5:
+                    lo, hi = (int(wrote[1] or wrote[2]), int(wrote[1] or wrote[3]))
+                    if sgprs & set(range(lo, hi + 1)):
+                        early.append((prev, op))
+                nop = re.match(r"s_nop (\d+)", prev)
+                waited += int(nop[1]) + 1 if nop else 1
+    assert dmas > 500                    # every DMA kernel was seen
+    assert not early, f"{len(early)} of {dmas}: {early[:3]}"
+
+
 def test_argument_validation_without_device(capi):
     lib = capi.load()
     P = ctypes.c_void_p

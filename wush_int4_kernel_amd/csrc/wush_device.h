@@ -305,18 +305,21 @@ __device__ __forceinline__ uint32_t lds_addr(const void* l) {
 // The compiler does not count these in its vmcnt waits: a caller waits for
 // them itself (WUSH_WAIT_VMCNT) and keeps its own LDS reads of the target in
 // order (sched_barrier, or the memory clobber of dma16_ordered).
+// The s_nop is the wait state that the hardware needs between a scalar write
+// of M0 and an LDS DMA reading it (without it the DMA may land at the address
+// of the one before); the compiler puts none inside an asm string.
 __device__ __forceinline__ void dma16(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(lds) : "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(lds) : "m0");
 }
 // the same from a wave-uniform base plus a 32-bit lane offset
 __device__ __forceinline__ void dma16_uniform(const void* base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds) : "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds) : "m0");
 }
 __device__ __forceinline__ void dma4(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(lds) : "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(lds) : "m0");
 }
 __device__ __forceinline__ void dma16_ordered(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(lds) : "m0", "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(lds) : "m0", "memory");
 }
 
 // s_waitcnt vmcnt(n) (n < 64) with the other counters left alone, and a
