@@ -141,6 +141,25 @@ int wush_gemm_s4(const uint8_t *xq, const uint16_t *xs, const uint8_t *wq, const
                  uint16_t *y, int64_t M, int64_t N, int64_t K,
                  void *workspace, size_t workspace_bytes, hipStream_t stream);
 
+/* Kernels of the GEMM entry points, as the two plan queries name them. */
+enum wush_gemm_kernel {
+    WUSH_GEMM_INT8_TILES = 0,       /* int8 MFMA tiles through LDS */
+    WUSH_GEMM_INT8_STREAM = 1,      /* int8 MFMA, weights streamed (M <= 64) */
+    WUSH_GEMM_FP16_TILES = 2,       /* fp16 MFMA tiles, operands converted per tile */
+    WUSH_GEMM_FP16_CONVERTED = 3,   /* fp16 MFMA tiles on activations converted into the workspace */
+    WUSH_GEMM_FP16_STREAM = 4,      /* fp16 MFMA, weights streamed (32 < M <= 64) */
+    WUSH_GEMM_TENSOR_TILES = 5      /* per-tensor int8 MFMA tiles */
+};
+
+/* The plan wush_gemm_s4 runs for (M, N, K) with 16-byte aligned operands and
+ * `workspace_bytes` of 16-byte aligned workspace: plan = {kernel, output rows
+ * of a workgroup, columns, K slices}.  Host only, no device is touched; for
+ * tests and tuning.  The reference has no counterpart. */
+int wush_gemm_s4_plan(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int32_t plan[4]);
+
+/* The same for wush_gemm_s4_tensor_scale. */
+int wush_gemm_s4_tensor_scale_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]);
+
 /* Bytes of the static split-K scratch that wush_gemm_s4_noalloc uses: one
  * array per device, held from the library's load until the process ends. */
 #define WUSH_GEMM_SCRATCH_BYTES (64u << 20)

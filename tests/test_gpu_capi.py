@@ -1164,14 +1164,20 @@ def test_per_tensor_quant_and_gemm(capi):
         assert np.array_equal(f16_tensor_f64(y), f16_tensor_f64(y2))
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 33, 256), (127, 129, 256), (128, 256, 512), (129, 1001, 768), (300, 2050, 1024),
-                                   (700, 3001, 768), (1025, 4100, 1280), (260, 24580, 512), (4000, 4104, 256),
-                                   (9, 65536, 256)])
-def test_per_tensor_tiles_exact(capi, M, N, K):
+@pytest.mark.parametrize("M,N,K,tile", [
+    (1, 33, 256, (128, 128)), (127, 129, 256, (128, 128)), (128, 256, 512, (128, 128)), (129, 1001, 768, (128, 128)),
+    (300, 2050, 1024, (128, 128)), (700, 3001, 768, (128, 128)), (260, 24580, 512, (128, 128)),
+    (4000, 4104, 256, (128, 128)), (1025, 4100, 1280, (256, 128)), (1025, 4099, 1280, (256, 128)),
+    (1020, 4104, 1280, (256, 128)), (509, 24577, 1024, (256, 256)), (1000, 12290, 2048, (256, 256)),
+    (510, 24584, 1024, (256, 256)), (9, 65536, 256, None)])
+def test_per_tensor_tiles_exact(capi, M, N, K, tile):
     # per-tensor tiles (K % 256 == 0) of every size and their edges, the
-    # 2-, 4- and 16-byte stores, one super-stage of K and more; codes over all
+    # 2-, 4- and 16-byte stores, one super-stage of K and more (and the int8
+    # tiles of few rows on wide weights: None); codes over all
     # of [-8, 7].  The int32 sum is exact and rounded once to fp16, so outputs
     # equal fp16(fp32(dot) * alpha) bit for bit, for aligned and unaligned y.
+    plan = capi.gemm_s4_tensor_scale_plan(M, N, K)
+    assert plan[0] == (capi.TENSOR_TILES if tile else capi.INT8_TILES) and (tile is None or plan[1:3] == tile)
     import torch
     g = rng(6200 + M + N)
     xq, wq = pack_codes(g.integers(-8, 8, (M, K))), pack_codes(g.integers(-8, 8, (N, K)))
@@ -1220,6 +1226,23 @@ def test_per_tensor_largest_k(capi):
     assert rel_fro(f16_tensor_f64(y), ref) < FRO_TOL
     with pytest.raises(RuntimeError, match="invalid argument"):
         c.gemm_s4_tensor_scale(dx.data_ptr(), dw.data_ptr(), y.data_ptr(), M, N, K + 32, 1.0, None, _stream())
+
+
+@pytest.mark.parametrize("M,N,tile", [(4, 64, (128, 128)), (4080, 4088, (256, 256))])
+def test_per_tensor_tiles_largest_k(capi, M, N, tile):
+    # the largest K of the per-tensor tiles, codes of -8 throughout: every
+    # int32 accumulator ends at its extreme, 256 * 64 * K
+    import torch
+    K = 130816
+    assert K % 256 == 0 and K + 256 > 131040
+    assert capi.gemm_s4_tensor_scale_plan(M, N, K) == (capi.TENSOR_TILES, *tile, 1)
+    dx = torch.full((M, K // 2), 0x88, dtype=torch.uint8, device="cuda")
+    dw = torch.full((N, K // 2), 0x88, dtype=torch.uint8, device="cuda")
+    y = torch.empty(M, N, dtype=torch.float16, device="cuda")
+    alpha = 2.0 ** -14
+    capi.gemm_s4_tensor_scale(dx.data_ptr(), dw.data_ptr(), y.data_ptr(), M, N, K, alpha, None, _stream())
+    torch.cuda.synchronize()
+    assert (y == float(np.float16(64.0 * K * alpha))).all()
 
 
 def test_invalid_arguments_rejected(capi):

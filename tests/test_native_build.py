@@ -149,6 +149,31 @@ def test_best_workspace_bytes_against_the_base(capi):
         assert best > capi.gemm_s4_workspace_bytes(M, N, K) and best >= 2 * M * K, (M, N, K)
 
 
+def test_plan_queries_are_host_only(capi):
+    # the kernel, tile and K slices a call runs, at the workspace it is given
+    def plan(M, N, K, ws):
+        return capi.gemm_s4_plan(M, N, K, ws)
+    shape = (203, 8195, 8192)
+    need = capi.gemm_s4_workspace_bytes(*shape)
+    kernel, rows, cols, splits = plan(*shape, need)
+    assert (kernel, cols) == (capi.FP16_CONVERTED, 256) and rows in (64, 128, 256)
+    # exactly what that plan holds: partials, then activations and shifts
+    partial = (splits * 203 * 8195 * 4 if splits > 1 else 0) + 255 & ~255
+    assert need == partial + 256 * 8192 * 2 + splits * (256 + 8448) * 4
+    assert plan(*shape, 0)[0] != capi.FP16_CONVERTED
+    assert plan(16, 4096, 4096, 0) == (capi.INT8_STREAM, 32, 32, 1)
+    assert plan(64, 57344, 8192, 0)[0] == capi.FP16_STREAM
+    assert plan(4096, 4096, 4096, 0) == (capi.FP16_TILES, 256, 256, 1)
+    assert plan(100, 64, 96, 0)[0] == capi.INT8_TILES
+    assert capi.gemm_s4_tensor_scale_plan(512, 24576, 4096)[0] == capi.TENSOR_TILES
+    assert capi.gemm_s4_tensor_scale_plan(64, 96, 96)[0] == capi.INT8_TILES
+    for bad in [(0, 64, 64), (4, 0, 64), (4, 64, 40)]:
+        with pytest.raises(RuntimeError, match="invalid argument"):
+            capi.gemm_s4_plan(*bad, 0)
+        with pytest.raises(RuntimeError, match="invalid argument"):
+            capi.gemm_s4_tensor_scale_plan(*bad)
+
+
 def test_torch_module_exposes_reference_ops():
     from my_int4 import _C
     import my_int4

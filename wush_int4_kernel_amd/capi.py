@@ -26,6 +26,8 @@ SIGNATURES = {
     "wush_gemv_int4_supported": ([_I64, _I64, _I64], _I),
     "wush_gemm_s4_workspace_bytes": ([_I64, _I64, _I64], _SZ),
     "wush_gemm_s4_best_workspace_bytes": ([_I64, _I64, _I64], _SZ),
+    "wush_gemm_s4_plan": ([_I64, _I64, _I64, _SZ, ctypes.POINTER(ctypes.c_int32)], _I),
+    "wush_gemm_s4_tensor_scale_plan": ([_I64, _I64, _I64, ctypes.POINTER(ctypes.c_int32)], _I),
     "wush_gemm_s4": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _SZ, _P], _I),
     "wush_gemm_s4_noalloc": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _I),
     "wush_mfma_selftest": ([_P, _P, _P, _P], _I),
@@ -85,6 +87,23 @@ def gemm_s4_workspace_bytes(M, N, K) -> int:
 
 def gemm_s4_best_workspace_bytes(M, N, K) -> int:
     return int(load().wush_gemm_s4_best_workspace_bytes(M, N, K))
+
+
+# kernels of gemm_s4_plan and gemm_s4_tensor_scale_plan
+INT8_TILES, INT8_STREAM, FP16_TILES, FP16_CONVERTED, FP16_STREAM, TENSOR_TILES = range(6)
+
+
+def gemm_s4_plan(M, N, K, workspace_bytes) -> tuple:
+    """(kernel, rows, columns, K slices) of gemm_s4 with that much workspace."""
+    plan = (ctypes.c_int32 * 4)()
+    _check(load().wush_gemm_s4_plan(M, N, K, workspace_bytes, plan), "wush_gemm_s4_plan")
+    return tuple(plan)
+
+
+def gemm_s4_tensor_scale_plan(M, N, K) -> tuple:
+    plan = (ctypes.c_int32 * 4)()
+    _check(load().wush_gemm_s4_tensor_scale_plan(M, N, K, plan), "wush_gemm_s4_tensor_scale_plan")
+    return tuple(plan)
 
 
 def gemm_s4(xq, xs, wq, ws, y, M, N, K, workspace, workspace_bytes, stream) -> None:

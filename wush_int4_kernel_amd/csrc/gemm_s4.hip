@@ -1048,6 +1048,20 @@ static void launch_stream32(dim3 grid, bool wide, const uint8_t* xq, const uint1
     }
 }
 
+// The plan of a call with `room` bytes of workspace (make_plan's arguments).
+template <bool PT>
+static Plan choose_plan(int64_t M, int64_t N, int64_t K, size_t room, bool scales16, bool allow_a16) {
+    bool narrow_a16 = false;
+    if (!PT && allow_a16 && N < WUSH_H16A_MIN_N && room > 0 && h16a_preferred(M, N, K))
+        narrow_a16 = room >= best_bytes(M, N, K, base_bytes(M, N, K));
+    return make_plan(M, N, K, room, !PT, scales16, allow_a16, narrow_a16);
+}
+
+static int plan_kernel(const Plan& p) {
+    if (p.cfg == 5) return p.a16 ? WUSH_GEMM_FP16_CONVERTED : WUSH_GEMM_FP16_TILES;
+    return p.cfg == 6 ? WUSH_GEMM_FP16_STREAM : p.cfg == 4 ? WUSH_GEMM_INT8_STREAM : WUSH_GEMM_INT8_TILES;
+}
+
 template <bool PT>
 static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
                     uint16_t* y, int64_t M, int64_t N, int64_t K, void* workspace, size_t ws_bytes,
@@ -1061,11 +1075,7 @@ static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, co
         if (plan_pt(M, N, K, &rows, &cols))
             return launch_gemm_pt(xq, wq, y, (int)M, (int)N, (int)K, alpha, alpha_dev, rows, cols, stream);
     }
-    const size_t room = workspace ? ws_bytes : 0;
-    bool narrow_a16 = false;
-    if (!PT && allow_a16 && N < WUSH_H16A_MIN_N && room > 0 && h16a_preferred(M, N, K))
-        narrow_a16 = room >= best_bytes(M, N, K, base_bytes(M, N, K));
-    const Plan p = make_plan(M, N, K, room, !PT, scales16, allow_a16, narrow_a16);
+    const Plan p = choose_plan<PT>(M, N, K, workspace ? ws_bytes : 0, scales16, allow_a16);
     WUSH_REQUIRE((N + p.tn - 1) / p.tn <= 0x7fffffffLL && (M + p.tm - 1) / p.tm <= 65535);
     float* partial = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     const int m = (int)M, n = (int)N, k = (int)K;
@@ -1127,6 +1137,30 @@ size_t wush_gemm_s4_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 size_t wush_gemm_s4_best_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 32) return 0;
     return wush::best_bytes(M, N, K, wush::base_bytes(M, N, K));
+}
+
+int wush_gemm_s4_plan(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int32_t plan[4]) {
+    WUSH_REQUIRE(M > 0 && N > 0 && K > 0 && K % 32 == 0 && plan);
+    WUSH_REQUIRE(M <= 0x7fffffffLL && N <= 0x7fffffffLL && K <= 0x7fffffffLL);
+    const wush::Plan p = wush::choose_plan<false>(M, N, K, workspace_bytes, true, true);
+    const int32_t v[4] = {wush::plan_kernel(p), p.tm, p.tn, p.splits};
+    std::copy(v, v + 4, plan);
+    return (int)hipSuccess;
+}
+
+int wush_gemm_s4_tensor_scale_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]) {
+    WUSH_REQUIRE(M > 0 && N > 0 && K > 0 && K % 32 == 0 && plan);
+    WUSH_REQUIRE(M <= 0x7fffffffLL && N <= 0x7fffffffLL && K <= WUSH_TENSOR_SCALE_MAX_K);
+    int rows = 0, cols = 0;
+    if (wush::plan_pt(M, N, K, &rows, &cols)) {
+        const int32_t v[4] = {WUSH_GEMM_TENSOR_TILES, rows, cols, 1};
+        std::copy(v, v + 4, plan);
+        return (int)hipSuccess;
+    }
+    const wush::Plan p = wush::choose_plan<true>(M, N, K, 0, false, false);
+    const int32_t v[4] = {wush::plan_kernel(p), p.tm, p.tn, p.splits};
+    std::copy(v, v + 4, plan);
+    return (int)hipSuccess;
 }
 
 int wush_gemm_s4(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
