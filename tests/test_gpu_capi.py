@@ -960,6 +960,71 @@ def test_gemm_h16q_ragged_columns(capi, M, N, K):
     assert (np.abs(got - ref) <= bound).all(), (M, N, K, float((np.abs(got - ref) / bound).max()))
 
 
+# (rows of a tile, K slices) of the plan in the last column
+H16Q_WIDE_SHAPES = [(131, 8198, 8192, (64, 2)), (1000, 2051, 2304, (64, 1)), (129, 6146, 6144, (128, 4)),
+                    (1030, 4096, 2048, (128, 1)), (203, 8195, 8192, (256, 4)), (2047, 4100, 2048, (256, 1)),
+                    (70, 7000, 12352, (64, 4)), (130, 16390, 4288, (64, 1)), (256, 4100, 8384, (128, 4)),
+                    (3000, 2050, 1088, (128, 1)), (203, 8195, 8256, (256, 4))]
+
+
+@pytest.mark.parametrize("M,N,K,plan", H16Q_WIDE_SHAPES)
+def test_gemm_h16q_wide_scales(capi, M, N, K, plan):
+    # Converted-activation tiles of every height, with and without a K split
+    # and a short last block: rows and columns whose scales span more than the
+    # fp16 operands hold (2^29 within a K slice) lose nothing.  The spanning
+    # group's codes are 0 on one side, so that the small groups make the
+    # output: every sampled output is within one fp16 rounding plus 2K rounded
+    # fp32 additions of the fp64 product, which flushed scales would miss.
+    import torch
+    wsb = capi.gemm_s4_best_workspace_bytes(M, N, K)
+    assert capi.gemm_s4_plan(M, N, K, wsb) == (capi.FP16_CONVERTED, plan[0], 256, plan[1])
+    g = rng(5100 + M + N)
+    G = K // 32
+    xq, xs, wq, ws = _rand_operands(g, M, N, K)
+    cx, cw = unpack_codes(xq), unpack_codes(wq)
+
+    def widen(codes, scales, i, grp, k, clear=True):     # group grp of row i: 2^k above the row's largest
+        scales[i, grp] = _bf16_times_pow2(scales[i].max(), k)
+        if clear:
+            codes[i, 32 * grp:32 * grp + 32] = 0
+    first, mid, last = 0, G // 2, G - 1
+    widen(cx, xs, 0, first, 100)
+    widen(cx, xs, 1, last, 31)
+    widen(cx, xs, M // 2, mid, 60)
+    widen(cx, xs, M - 1, mid, 100)
+    widen(cx, xs, M - 1, first, 20)
+    widen(cw, ws, 0, last, 100)
+    widen(cw, ws, 255, mid, 31)
+    widen(cw, ws, 256, first, 60)
+    widen(cw, ws, N - 1, first, 100)
+    # a row whose spanning group has codes; columns with none there stay finite
+    widen(cx, xs, 2, 3, 90, clear=False)
+    zero = np.array([7, N // 2, N - 3])
+    cw[zero, 96:128] = 0
+    # a row and a column whose tiny scales carry no codes: nothing to lose
+    xs[3, 5:9], cx[3, 160:288] = 0x0080, 0
+    ws[9, 5:9], cw[9, 160:288] = 0x0080, 0
+    # a non-finite row and column across them
+    xs[4, G - 2], ws[11, 1] = 0x7F80, 0xFFC0
+    xq, wq = pack_codes(cx), pack_codes(cw)
+    d = _dev_operands(xq, xs, wq, ws)
+    work = torch.full((wsb,), 0xFF, dtype=torch.uint8, device="cuda")
+    yt = torch.empty(M, N, dtype=torch.float16, device="cuda")
+    capi.gemm_s4(*[t.data_ptr() for t in d], yt.data_ptr(), M, N, K, work.data_ptr(), wsb, _stream())
+    torch.cuda.synchronize()
+    y = f16_tensor_f64(yt)
+    assert np.isnan(y[4]).all() and np.isnan(y[:, 11]).all()
+    wide_r, wide_c = [0, 1, 3, M // 2, M - 1], [0, 9, 255, 256, N - 1]
+    for rows, cols in ((wide_r, _sample(g, N, 300)), (_sample(g, M, 40), wide_c), ([2], zero)):
+        rows = np.array([r for r in rows if r != 4 and (r != 2 or cols is zero)])
+        cols = np.array([c for c in cols if c != 11])
+        ref = oracle.gemm_f64(xq[rows], xs[rows], wq[cols], ws[cols])
+        A = _abs_product(xq[rows], xs[rows], wq[cols], ws[cols])
+        bound = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64) + 2 * K * 2.0 ** -24 * A + 2.0 ** -25
+        got = y[np.ix_(rows, cols)]
+        assert (np.abs(got - ref) <= bound).all(), (M, N, K, float((np.abs(got - ref) / bound).max()))
+
+
 # Narrow weights (N < 8192): every tile height (64, 128, 256 rows) and K splits
 # from 1 to 16, ragged M and N, K that is a multiple of 64 only (the last
 # block of 8 groups holds 2, 4 or 6), splits of unequal length

@@ -26,7 +26,9 @@ int launch_gemm_h16(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, co
 // first kernel (with every weight column's shift), then DMA'd into LDS by the
 // GEMM kernel (gemm_h16q.hip).  The same fp16 operands as launch_gemm_h16,
 // summed in another K order within blocks of four groups: equal to fp32
-// rounding.  K % 64 == 0 (the last 8 groups may be short); needs 16-byte
+// rounding, except that rows and columns whose scales span more than those
+// operands hold (2^29 within a K slice) are computed apart and lose nothing.
+// K % 64 == 0 (the last 8 groups may be short); needs 16-byte
 // aligned scale tensors.  tile_rows: rows of an
 // output tile (256 columns wide), 64, 128 or 256.
 size_t gemm_h16a_workspace_bytes(int64_t M, int64_t N, int64_t K, int splits);

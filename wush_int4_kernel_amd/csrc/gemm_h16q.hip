@@ -47,6 +47,11 @@
 // with per-output tests and 2-byte writes a 256 x 256 tile spent 15-20 us
 // outside its K loop, now about 10.
 //
+// Rows and columns whose scales span more than the operands hold (h16_loses_bits)
+// are found by the conversion kernel, and a tile ends by computing their
+// outputs from the codes and bf16 scales: nothing is paid for inputs without
+// them but one test per row and column.
+//
 // Measured (layer with the fused transform, same box, against the 32x32x16
 // form with burst DMAs): K=8192 N=57344 M=4096 3179 -> 2679 us (1.45 PFLOP/s;
 // a library fp16 GEMM of the shape 2560-2850), M=256 238 -> 197, M=128 146 ->
@@ -60,6 +65,41 @@ namespace wush {
 namespace {
 
 constexpr int kH16qStage = kH16Tile * 64;        // workspace bytes of one stage of a 256-row tile
+// Row/column shift marking codes whose scale loses bits as a shifted fp16
+// operand: it is more than 2^29 below the row's largest over the K slice (the
+// largest lies in [2^12, 2^13), fp16's lowest bit is 2^-24, a bf16 has 8).
+constexpr int kH16Wide = 1 << 21;
+
+__device__ __forceinline__ bool h16_loses_bits(uint32_t bits, uint32_t mx) {
+    return (int)(mx >> 7) - max((int)(bits >> 7), 1) > 29;
+}
+
+// Output (m, n) over groups [g0, g1) from the codes and bf16 scales: exact
+// int32 group dots summed in fp64.  For the outputs of wide rows and columns
+// only: such inputs are rare, so one lane per output, unblocked, will do.
+__device__ __forceinline__ float h16_exact_output(const uint8_t* __restrict__ xq, const uint16_t* __restrict__ xs,
+                                                  const uint8_t* __restrict__ wq, const uint16_t* __restrict__ ws,
+                                                  int m, int n, int GR, int g0, int g1) {
+    const uint4* x = reinterpret_cast<const uint4*>(xq + (size_t)m * GR * 16);
+    const uint4* w = reinterpret_cast<const uint4*>(wq + (size_t)n * GR * 16);
+    const uint16_t* sx = xs + (size_t)m * GR;
+    const uint16_t* sw = ws + (size_t)n * GR;
+    double acc = 0.0;
+#pragma unroll 1
+    for (int g = g0; g < g1; ++g) {
+        const uint4 a = x[g], b = w[g];
+        int d = __builtin_amdgcn_sdot8((int)a.x, (int)b.x, 0, false);
+        d = __builtin_amdgcn_sdot8((int)a.y, (int)b.y, d, false);
+        d = __builtin_amdgcn_sdot8((int)a.z, (int)b.z, d, false);
+        d = __builtin_amdgcn_sdot8((int)a.w, (int)b.w, d, false);
+        const uint32_t ux = sx[g], uw = sw[g];
+        // a non-finite scale makes its row or column NaN whatever the codes
+        if (max(ux & 0x7fffu, uw & 0x7fffu) >= 0x7f80u) return __builtin_nanf("");
+        acc += (double)d * (double)__uint_as_float(ux << 16) * (double)__uint_as_float(uw << 16);
+    }
+    return (float)acc;
+}
+
 // RB: 16-row blocks per wavefront, 16 (256-row tiles) or 8 (128-row tiles:
 // half the accumulators, the same weight conversion per stage) or 4.  PAD: K is
 // a multiple of 64 but not of 256: the last double batch reads the row's last
@@ -70,7 +110,8 @@ template <int RB, bool PAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ ea, const int* __restrict__ eb,
                       const uint8_t* __restrict__ wq, const uint16_t* __restrict__ ws, uint16_t* __restrict__ y,
-                      float* __restrict__ partial, int M, int N, int K, int groups_per_split) {
+                      float* __restrict__ partial, int M, int N, int K, int groups_per_split,
+                      const uint8_t* __restrict__ xq, const uint16_t* __restrict__ xs) {
     constexpr int TR = 16 * RB, TC = kH16Tile;
     constexpr int NA = TR / 64;                  // activation DMAs per wavefront and stage
     constexpr int NM = 4 * RB;                   // MFMAs per stage
@@ -271,12 +312,16 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
     asm volatile("s_nop 15\n\ts_nop 15");        // the last MFMAs' results
     __syncthreads();                             // the ring is free
 
+    // the lane number again: kept over the loop, what derives from it would
+    // spill a register of the 256-row tile
+    const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const int lr = ln & 15, lq = ln >> 4;
     const int wn0 = n0 + wave * 64;
     int er[RB];
 #pragma unroll
-    for (int i = 0; i < RB; ++i) er[i] = sh_e[i * 16 + l16];
-    const int4* ec4 = reinterpret_cast<const int4*>(sh_e + 256 + wave * 64 + 4 * kq);
-    // accumulator [i][j][q]: row 16 i + l16, column 16 j + 4 kq + q
+    for (int i = 0; i < RB; ++i) er[i] = sh_e[i * 16 + lr];
+    const int4* ec4 = reinterpret_cast<const int4*>(sh_e + 256 + wave * 64 + 4 * lq);
+    // accumulator [i][j][q]: row 16 i + lr, column 16 j + 4 lq + q
     auto out4 = [&](int i, int j, const int4& ec) {
         v4f v;
         v[0] = __builtin_ldexpf(acc[i][j][0], er[i] + ec.x);
@@ -285,20 +330,18 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
         v[3] = __builtin_ldexpf(acc[i][j][3], er[i] + ec.w);
         return v;
     };
-    // columns with a non-finite scale (one per lane): NaN over what was stored
-    uint64_t bad = __ballot(sh_e[256 + wave * 64 + lane] == kH16NonFinite);
     if (partial != nullptr) {
         // fp32 partials of a K slice, 64 contiguous bytes per row and instruction
         const bool vec = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(partial) & 15u) == 0;
-        float* prow = partial + ((size_t)slice * M + m0 + l16) * N + wn0 + 4 * kq;
+        float* prow = partial + ((size_t)slice * M + m0 + lr) * N + wn0 + 4 * lq;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int4 ec = ec4[j * 4];
-            const int n = wn0 + j * 16 + 4 * kq;
+            const int n = wn0 + j * 16 + 4 * lq;
 #pragma unroll
             for (int i = 0; i < RB; ++i) {
                 const v4f v = out4(i, j, ec);
-                if (m0 + i * 16 + l16 < M) {
+                if (m0 + i * 16 + lr < M) {
                     float* dst = prow + (size_t)(i * 16) * N + j * 16;
                     if (vec) {
                         if (n < N) *reinterpret_cast<v4f*>(dst) = v;
@@ -311,64 +354,79 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (bad != 0) {
-            WUSH_WAIT_VMCNT(0);
-            for (; bad != 0; bad &= bad - 1) {
-                const int n = wn0 + __builtin_ctzll(bad);
-                for (int m = m0 + lane; m < min(M, m0 + TR); m += 64)
-                    if (n < N) partial[((size_t)slice * M + m) * N + n] = __builtin_nanf("");
-            }
-        }
-        return;
-    }
-    // fp16: each wavefront's TR x 64 outputs through LDS, 128 bytes a row,
-    // 16-byte chunk c of row r at chunk c ^ (r % 8)
-    uint8_t* stg = smem + wave * (TR * 128);
-    uint8_t* wst = stg + l16 * 128 + (kq & 1) * 8;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int4 ec = ec4[j * 4];
-        uint8_t* w = wst + ((j * 2 + (kq >> 1)) ^ (l16 & 7)) * 16;
-#pragma unroll
-        for (int i = 0; i < RB; ++i)
-            *reinterpret_cast<h4*>(w + i * 16 * 128) = __builtin_convertvector(out4(i, j, ec), h4);
-        __builtin_amdgcn_sched_barrier(0);       // one column block at a time
-    }
-    const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-    // the lane number again: kept from the start it would spill a register
-    const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    if (vec) {
-        const int r0 = ln >> 3, cc = ln & 7;
-        const int n = wn0 + cc * 8;
-        const uint8_t* rst = stg + r0 * 128 + (cc ^ r0) * 16;    // row 8 k + r0: (8 k + r0) % 8 == r0
-        uint16_t* yrow = y + (size_t)(m0 + r0) * N + n;
-#pragma unroll
-        for (int k = 0; k < TR / 8; ++k) {
-            const uint4 v = *reinterpret_cast<const uint4*>(rst + k * 1024);
-            if (m0 + 8 * k + r0 < M && n < N) *reinterpret_cast<uint4*>(yrow + (size_t)(8 * k) * N) = v;
-        }
-    } else if ((N & 1) == 0 && (reinterpret_cast<uintptr_t>(y) & 3u) == 0) {
-        store_staged<128, uint32_t>(stg, TR, y, m0, M, wn0, N, ln);
     } else {
-        store_staged<128, uint16_t>(stg, TR, y, m0, M, wn0, N, ln);
-    }
-    if (bad != 0) {
-        WUSH_WAIT_VMCNT(0);
-        for (; bad != 0; bad &= bad - 1) {
-            const int c = wn0 + __builtin_ctzll(bad);
-            for (int m = m0 + lane; m < min(M, m0 + TR); m += 64)
-                if (c < N) y[(size_t)m * N + c] = 0x7e00;
+        // fp16: each wavefront's TR x 64 outputs through LDS, 128 bytes a row,
+        // 16-byte chunk c of row r at chunk c ^ (r % 8)
+        uint8_t* stg = smem + wave * (TR * 128);
+        uint8_t* wst = stg + lr * 128 + (lq & 1) * 8;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int4 ec = ec4[j * 4];
+            uint8_t* w = wst + ((j * 2 + (lq >> 1)) ^ (lr & 7)) * 16;
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+                *reinterpret_cast<h4*>(w + i * 16 * 128) = __builtin_convertvector(out4(i, j, ec), h4);
+            __builtin_amdgcn_sched_barrier(0);       // one column block at a time
+        }
+        const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+        if (vec) {
+            const int r0 = ln >> 3, cc = ln & 7;
+            const int n = wn0 + cc * 8;
+            const uint8_t* rst = stg + r0 * 128 + (cc ^ r0) * 16;    // row 8 k + r0: (8 k + r0) % 8 == r0
+            uint16_t* yrow = y + (size_t)(m0 + r0) * N + n;
+#pragma unroll
+            for (int k = 0; k < TR / 8; ++k) {
+                const uint4 v = *reinterpret_cast<const uint4*>(rst + k * 1024);
+                if (m0 + 8 * k + r0 < M && n < N) *reinterpret_cast<uint4*>(yrow + (size_t)(8 * k) * N) = v;
+            }
+        } else if ((N & 1) == 0 && (reinterpret_cast<uintptr_t>(y) & 3u) == 0) {
+            store_staged<128, uint32_t>(stg, TR, y, m0, M, wn0, N, ln);
+        } else {
+            store_staged<128, uint16_t>(stg, TR, y, m0, M, wn0, N, ln);
         }
     }
+    // Over what was stored: outputs of wide rows and columns, then NaN for the
+    // columns with a non-finite scale.
+    auto put = [&](int m, int n, float v) {
+        if (m >= M || n >= N) return;
+        if (partial != nullptr) partial[((size_t)slice * M + m) * N + n] = v;
+        else reinterpret_cast<_Float16*>(y)[(size_t)m * N + n] = (_Float16)v;
+    };
+    const int ecl = sh_e[256 + wave * 64 + ln];     // one column per lane
+    uint64_t bad = __ballot(ecl == kH16NonFinite), wide = __ballot(ecl == kH16Wide);
+    const int g1 = min(GR, gb + groups_per_split);
+    bool waited = false;
+    for (; wide != 0; wide &= wide - 1) {
+        if (!waited) WUSH_WAIT_VMCNT(0);
+        waited = true;
+        const int n = wn0 + __builtin_ctzll(wide);
+        for (int m = m0 + ln; m < min(M, m0 + TR); m += 64)
+            put(m, n, h16_exact_output(xq, xs, wq, ws, m, n, GR, gb, g1));
+    }
+    for (int r = 0; r < TR; r += 64) {
+        for (wide = __ballot(sh_e[r + ln] == kH16Wide); wide != 0; wide &= wide - 1) {
+            if (!waited) WUSH_WAIT_VMCNT(0);
+            waited = true;
+            const int m = m0 + r + __builtin_ctzll(wide);
+            const int n = wn0 + ln;
+            if (n < N) put(m, n, h16_exact_output(xq, xs, wq, ws, m, n, GR, gb, g1));
+        }
+    }
+    if (bad != 0) WUSH_WAIT_VMCNT(0);
+    for (; bad != 0; bad &= bad - 1)
+        for (int m = m0 + ln; m < min(M, m0 + TR); m += 64)
+            put(m, wn0 + __builtin_ctzll(bad), __builtin_nanf(""));
 }
 
 // ------------------------------------------------ pre-converted activations
 // a16 layout: [256-row tile][stage][16-row block][64 lanes][16 B]; stage
 // 4b + s, lane (row % 16) + 16 q holds the 8 fp16 operands of dword s of group
 // 4b + q.  ea[slice][row] and eb[slice][column] hold MINUS the power-of-two
-// shift over the K slice, or kH16NonFinite for a column with a non-finite
-// scale (its outputs are set to NaN); a row with one gets NaN operands.
-// Rows past M are zero (shift 0 for them and for columns past N).
+// shift over the K slice, kH16NonFinite for a column with a non-finite scale
+// (its outputs are set to NaN; a row with one gets NaN operands), or kH16Wide
+// for a row or column with nonzero codes under a scale that would lose bits
+// (its outputs are computed apart).  Rows past M are zero (shift 0 for them
+// and for columns past N).
 //
 // Workgroups [0, na) convert 32 rows by `chunk` groups of one slice each
 // (scanning the rows' scales of the slice first, 8 threads a row); the rest
@@ -378,23 +436,37 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
 // with each thread loading 16 bytes of its own row and one 32-row block per
 // workgroup (most of a wave of workgroups idle at small M).
 // PAD: G % 8 != 0, so rows of scales are 4-byte aligned (G is even).
+//
+// Bits (sign cleared) of the largest scale, and of the smallest nonzero one
+// less 1 (0xffff: all are zero).
+struct ScaleRange {
+    uint32_t mx, mn;
+};
+
 template <bool PAD>
-__device__ __forceinline__ uint32_t slice_scale_max(const uint16_t* p, int n, int part) {
-    u16x2 m2 = {0, 0};
+__device__ __forceinline__ ScaleRange slice_scale_range(const uint16_t* p, int n, int part) {
+    u16x2 m2 = {0, 0}, n2 = {0xffff, 0xffff};
+    auto take = [&](uint32_t w) {
+        const u16x2 v = abs_bits2(w);
+        m2 = __builtin_elementwise_max(m2, v);
+        n2 = __builtin_elementwise_min(n2, (u16x2)(v - (u16x2){1, 1}));
+    };
     if constexpr (PAD) {
         const uint32_t* p1 = reinterpret_cast<const uint32_t*>(p);
 #pragma unroll 4
-        for (int i = part; i < (n >> 1); i += 8) m2 = __builtin_elementwise_max(m2, abs_bits2(p1[i]));
-        return max((uint32_t)m2.x, (uint32_t)m2.y);
-    }
-    const uint4* p4 = reinterpret_cast<const uint4*>(p);
+        for (int i = part; i < (n >> 1); i += 8) take(p1[i]);
+    } else {
+        const uint4* p4 = reinterpret_cast<const uint4*>(p);
 #pragma unroll 4
-    for (int i = part; i < (n >> 3); i += 8) {
-        const uint4 v = p4[i];
-        m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(abs_bits2(v.x), abs_bits2(v.y)));
-        m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(abs_bits2(v.z), abs_bits2(v.w)));
+        for (int i = part; i < (n >> 3); i += 8) {
+            const uint4 v = p4[i];
+            take(v.x);
+            take(v.y);
+            take(v.z);
+            take(v.w);
+        }
     }
-    return max((uint32_t)m2.x, (uint32_t)m2.y);
+    return {max((uint32_t)m2.x, (uint32_t)m2.y), min((uint32_t)n2.x, (uint32_t)n2.y)};
 }
 
 constexpr int kPrepChunk = 32;                   // groups per converting workgroup
@@ -403,6 +475,7 @@ template <bool PAD>
 __global__ __launch_bounds__(256) void h16_prep_kernel(const uint8_t* __restrict__ xq,
                                                        const uint16_t* __restrict__ xs,
                                                        uint8_t* __restrict__ a16, int* __restrict__ ea,
+                                                       const uint8_t* __restrict__ wq,
                                                        const uint16_t* __restrict__ ws, int* __restrict__ eb,
                                                        int M, int N, int G, int groups_per_split, int mblocks,
                                                        int nblocks, int chunks, int na) {
@@ -417,18 +490,37 @@ __global__ __launch_bounds__(256) void h16_prep_kernel(const uint8_t* __restrict
     const int sg0 = slice * groups_per_split, sg1 = min(G, sg0 + groups_per_split);
     const int row = blk * 32 + r;
     const bool ok = row < (wside ? N : M);
-    uint32_t mx = ok ? slice_scale_max<PAD>((wside ? ws : xs) + (size_t)row * G + sg0, sg1 - sg0, part) : 0x3f80u;
-    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 1));
-    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 2));
-    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 4));
-    const int e = h16_shift(mx);
-    if (wside) {
-        if (part == 0) eb[(size_t)slice * (nblocks * 32) + row] = !ok ? 0 : e == kH16NonFinite ? kH16NonFinite : -e;
-        return;
+    const uint16_t* s = (wside ? ws : xs) + (size_t)row * G;
+    const uint8_t* q = (wside ? wq : xq) + (size_t)row * G * 16;
+    ScaleRange sr = {0x3f80u, 0xffffu};
+    if (ok) sr = slice_scale_range<PAD>(s + sg0, sg1 - sg0, part);
+#pragma unroll
+    for (int x = 1; x <= 4; x *= 2) {
+        sr.mx = max(sr.mx, (uint32_t)__shfl_xor((int)sr.mx, x));
+        sr.mn = min(sr.mn, (uint32_t)__shfl_xor((int)sr.mn, x));
     }
-    if (part == 0 && chunk == 0) ea[(size_t)slice * (mblocks * 32) + row] = !ok || e == kH16NonFinite ? 0 : -e;
-    const uint8_t* q = xq + (size_t)row * G * 16;
-    const uint16_t* s = xs + (size_t)row * G;
+    const int e = h16_shift(sr.mx);
+    if (wside || chunk == 0) {
+        int code = !ok ? 0 : e == kH16NonFinite ? (wside ? kH16NonFinite : 0) : -e;
+        if (e != kH16NonFinite && sr.mn != 0xffffu && h16_loses_bits(sr.mn + 1, sr.mx)) {
+            // a scale too small for the row's shift: wide unless its codes are 0
+            int wide = 0;
+            for (int g = sg0 + part; g < sg1; g += 8) {
+                const uint32_t bits = s[g] & 0x7fffu;
+                if (bits == 0 || !h16_loses_bits(bits, sr.mx)) continue;
+                const uint4 w = *reinterpret_cast<const uint4*>(q + (size_t)g * 16);
+                if ((w.x | w.y | w.z | w.w) != 0) wide = 1;
+            }
+#pragma unroll
+            for (int x = 1; x <= 4; x *= 2) wide |= __shfl_xor(wide, x);
+            if (wide) code = kH16Wide;
+        }
+        if (part == 0) {
+            if (wside) eb[(size_t)slice * (nblocks * 32) + row] = code;
+            else ea[(size_t)slice * (mblocks * 32) + row] = code;
+        }
+    }
+    if (wside) return;
     const int GP = PAD ? (G + 7) & ~7 : G;
     uint8_t* dst = a16 + (size_t)(blk >> 3) * GP * kH16qStage + (blk & 7) * 2048 + (r >> 4) * 1024 + (r & 15) * 16;
     const int g1 = min(min(GP, sg0 + groups_per_split), sg0 + (chunk + 1) * kPrepChunk);
@@ -481,14 +573,15 @@ int launch_gemm_h16a(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, c
     const long long tiles = (long long)((N + kH16Tile - 1) / kH16Tile) * ((M + tile_rows - 1) / tile_rows) * splits;
     if (nprep > 0x7fffffffLL || tiles > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     const auto prep = pad ? h16_prep_kernel<true> : h16_prep_kernel<false>;
-    prep<<<dim3((unsigned)nprep), 256, 0, stream>>>(xq, xs, a16, ea, ws, eb, M, N, G, groups_per_split, mblocks, nblocks,
+    prep<<<dim3((unsigned)nprep), 256, 0, stream>>>(xq, xs, a16, ea, wq, ws, eb, M, N, G, groups_per_split, mblocks, nblocks,
                                                     chunks, (int)na);
     const int e = (int)hipGetLastError();
     if (e != 0) return e;
     const auto kernel = tile_rows == 64    ? (pad ? gemm_h16q_kernel<4, true> : gemm_h16q_kernel<4, false>)
                         : tile_rows == 128 ? (pad ? gemm_h16q_kernel<8, true> : gemm_h16q_kernel<8, false>)
                                            : (pad ? gemm_h16q_kernel<16, true> : gemm_h16q_kernel<16, false>);
-    kernel<<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K, groups_per_split);
+    kernel<<<dim3((unsigned)tiles), 256, 0, stream>>>(a16, ea, eb, wq, ws, y, partial, M, N, K, groups_per_split, xq,
+                                                    xs);
     return (int)hipGetLastError();
 }
 
