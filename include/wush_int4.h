@@ -109,8 +109,10 @@ int wush_gemv_int4_supported(int64_t M, int64_t N, int64_t K);
 /* Bytes of workspace wush_gemm_s4 uses for (M, N, K); 0 when it needs none:
  * fp32 split-K partials, and for prefill shapes with N >= 8192 the
  * activations converted once to fp16 operands (M*K*2 bytes, padded to 256
- * rows and 256 of K).  A caller may pass a larger buffer; a smaller one makes wush_gemm_s4
- * choose a plan that needs no more than it is given (same results). */
+ * rows and 256 of K).  A caller may pass a larger buffer; a smaller one makes
+ * wush_gemm_s4 choose a plan that needs no more than it is given: another K
+ * split or another kernel, whose results agree within the tolerance below, not
+ * bit for bit. */
 size_t wush_gemm_s4_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* Bytes of workspace with which wush_gemm_s4 runs its fastest plan; at least
@@ -142,6 +144,19 @@ size_t wush_gemm_s4_best_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int wush_gemm_s4(const uint8_t *xq, const uint16_t *xs, const uint8_t *wq, const uint16_t *ws,
                  uint16_t *y, int64_t M, int64_t N, int64_t K,
                  void *workspace, size_t workspace_bytes, hipStream_t stream);
+
+/* wush_gemm_s4's plan for a workspace of wush_gemm_s4_best_workspace_bytes,
+ * run over `rows` activation rows at a time (a multiple of 64, or at least M)
+ * on a 16-byte aligned workspace of wush_gemm_s4_rows_workspace_bytes for the
+ * same operands and rows.  Every value of `rows` gives the same bits, those of
+ * that wush_gemm_s4 call: for callers short of memory that must not get other
+ * results for it.  Slower, the shorter the runs.  The reference has no
+ * counterpart. */
+size_t wush_gemm_s4_rows_workspace_bytes(const uint8_t *xq, const uint16_t *xs, const uint8_t *wq,
+                                         const uint16_t *ws, int64_t M, int64_t N, int64_t K, int64_t rows);
+int wush_gemm_s4_rows(const uint8_t *xq, const uint16_t *xs, const uint8_t *wq, const uint16_t *ws,
+                      uint16_t *y, int64_t M, int64_t N, int64_t K, int64_t rows,
+                      void *workspace, size_t workspace_bytes, hipStream_t stream);
 
 /* Kernels of the GEMM entry points, as the two plan queries name them. */
 enum wush_gemm_kernel {

@@ -663,6 +663,43 @@ def test_gemm_random_shapes_all_paths(capi):
         assert rel_fro(f16_tensor_f64(y3), ref) < FRO_TOL, (case, M, N, K, "unaligned scales")
 
 
+# converted-activation tiles (narrow and wide weights, split K, short last block,
+# ragged), int8 tiles with a K split, streaming kernels
+@pytest.mark.parametrize("M,N,K", [(1000, 2051, 2304), (203, 8195, 8192), (256, 4100, 8384), (700, 4099, 2240),
+                                   (130, 300, 4096), (40, 1000, 1024)])
+def test_gemm_rows_at_a_time_same_bits(capi, M, N, K):
+    # wush_gemm_s4_rows: the bits of the one-call plan for every number of rows
+    # at a time and for 2-byte aligned scales, within exactly the workspace it
+    # names
+    import torch
+    g = rng(4290 + M)
+    dx, dxs, dw, dws = _dev_operands(*_rand_operands(g, M, N, K))
+    best = capi.gemm_s4_best_workspace_bytes(M, N, K)
+    for off in (0, 1):
+        bx = torch.zeros(dxs.numel() + 8, dtype=torch.bfloat16, device="cuda")
+        bw = torch.zeros(dws.numel() + 8, dtype=torch.bfloat16, device="cuda")
+        bx[off:off + dxs.numel()] = dxs.reshape(-1)
+        bw[off:off + dws.numel()] = dws.reshape(-1)
+        args = dx.data_ptr(), bx.data_ptr() + 2 * off, dw.data_ptr(), bw.data_ptr() + 2 * off
+        work = torch.empty(max(best, 1), dtype=torch.uint8, device="cuda")
+        one = torch.empty(M, N, dtype=torch.float16, device="cuda")
+        capi.gemm_s4(*args, one.data_ptr(), M, N, K, work.data_ptr() if best else None, best, _stream())
+        for rows in (64, 128, 192, M, M + 1):
+            need = capi.gemm_s4_rows_workspace_bytes(*args, M, N, K, rows)
+            assert need <= best
+            buf = torch.full((need + 256,), 0xA5, dtype=torch.uint8, device="cuda")
+            y = torch.full((M * N + 8,), 7.0, dtype=torch.float16, device="cuda")
+            capi.gemm_s4_rows(*args, y.data_ptr(), M, N, K, rows, buf.data_ptr() if need else None, need, _stream())
+            torch.cuda.synchronize()
+            assert torch.equal(y[:M * N].view(M, N), one) and (y[M * N:] == 7.0).all(), (off, rows)
+            assert (buf[need:] == 0xA5).all(), (off, rows)
+            if need:
+                with pytest.raises(RuntimeError, match="invalid argument"):
+                    capi.gemm_s4_rows(*args, y.data_ptr(), M, N, K, rows, buf.data_ptr(), need - 1, _stream())
+    with pytest.raises(RuntimeError, match="invalid argument"):
+        capi.gemm_s4_rows(*args, y.data_ptr(), M, N, K, 33 if M > 33 else 0, None, 0, _stream())
+
+
 # Shapes the planner sends to the 256x256 fp16-MFMA tiles (K % 256 == 0,
 # M >= 256, at least 128 tiles): ragged M and N, one and several load batches.
 # The last two split K across workgroups (8 and 4 slices of 8 groups).

@@ -303,6 +303,52 @@ def test_rtn_int4_module_on_gpu(C):
     assert rel_fro(f16_tensor_f64(y.reshape(-1, 96)), ref) < 2e-3
 
 
+@pytest.mark.parametrize("M,N,K", [(2000, 4100, 16384), (1000, 8200, 16448)])
+def test_product_bits_do_not_depend_on_free_memory(C, M, N, K):
+    # with room for y but not for the workspace of all rows, the product runs
+    # the same plan over fewer rows at a time: the same bits; without room for
+    # 64 rows either it raises torch's out-of-memory error
+    import torch
+    from wush_int4_kernel_amd import capi
+    gen = torch.Generator(device="cuda").manual_seed(M)
+
+    def operand(rows):
+        q = torch.randint(0, 256, (rows, K // 2), generator=gen, device="cuda", dtype=torch.uint8)
+        return q, (torch.rand(rows, K // 32, generator=gen, device="cuda") * 0.02 + 0.001).to(torch.bfloat16)
+    (xq, xs), (wq, ws) = operand(M), operand(N)
+    want = C.w4a4_gemm_s4(xq, xs, wq, ws)
+    torch.cuda.synchronize()
+    full = capi.gemm_s4_best_workspace_bytes(M, N, K)
+    MiB = 1 << 20
+    y_room = (2 * M * N + 2 * MiB - 1) // (2 * MiB) * (2 * MiB)
+    filler = []
+
+    def leave_free(nbytes):      # in blocks of 2 MiB and more, beside what is reserved
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        try:
+            while True:
+                filler.append(torch.empty(2 * MiB, dtype=torch.uint8, device="cuda"))
+        except torch.OutOfMemoryError:
+            pass
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + nbytes) / total)
+    try:
+        leave_free(y_room + full * 2 // 3)
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        got = C.w4a4_gemm_s4(xq, xs, wq, ws)
+        torch.cuda.synchronize()
+        assert torch.cuda.max_memory_allocated() - before < y_room + full    # fewer rows at a time
+        assert torch.equal(got, want)
+        del got
+        leave_free(y_room + 2 * MiB)
+        with pytest.raises(torch.OutOfMemoryError):
+            C.w4a4_gemm_s4(xq, xs, wq, ws)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
 def test_s4_atom_selftest(C):
     import torch
     g = rng(7)

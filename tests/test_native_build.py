@@ -116,6 +116,13 @@ def test_argument_validation_without_device(capi):
     assert lib.wush_gemv_int4(P(16), P(16), P(16), P(16), P(16), 9, 4, 64, None) == INVALID  # M > 8
     assert lib.wush_gemv_int4(P(16), P(16), P(16), P(16), P(16), 8, 4, 1 << 20, None) == INVALID  # LDS
     assert lib.wush_gemm_s4(P(16), P(16), P(16), P(16), P(16), 4, 4, 40, None, 0, None) == INVALID
+    # rows at a time: a multiple of 64 or all of them, the workspace whole
+    assert lib.wush_gemm_s4_rows(None, None, None, None, None, 0, 8, 64, 64, None, 0, None) == 0
+    for M, rows in ((100, 33), (100, 0), (64, -64)):
+        assert lib.wush_gemm_s4_rows(P(16), P(16), P(16), P(16), P(16), M, 4, 64, rows, None, 0, None) == INVALID
+    need = lib.wush_gemm_s4_rows_workspace_bytes(P(16), P(16), P(16), P(16), 2048, 4096, 4096, 64)
+    assert 0 < need < lib.wush_gemm_s4_best_workspace_bytes(2048, 4096, 4096)
+    assert lib.wush_gemm_s4_rows(P(16), P(16), P(16), P(16), P(16), 2048, 4096, 4096, 64, P(16), need - 1, None) == INVALID
     assert lib.wush_gemm_s4_tensor_scale(P(16), P(16), P(16), 4, 4, 1 << 21, 1.0, None, None) == INVALID
     # int32 bound of the per-tensor GEMM: 256 * 64 * K < 2^31 for K <= 131040
     assert 256 * 64 * 131040 < 2 ** 31 <= 256 * 64 * (131040 + 32)

@@ -26,6 +26,8 @@ SIGNATURES = {
     "wush_gemv_int4_supported": ([_I64, _I64, _I64], _I),
     "wush_gemm_s4_workspace_bytes": ([_I64, _I64, _I64], _SZ),
     "wush_gemm_s4_best_workspace_bytes": ([_I64, _I64, _I64], _SZ),
+    "wush_gemm_s4_rows_workspace_bytes": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64], _SZ),
+    "wush_gemm_s4_rows": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _SZ, _P], _I),
     "wush_gemm_s4_plan": ([_I64, _I64, _I64, _SZ, ctypes.POINTER(ctypes.c_int32)], _I),
     "wush_gemm_s4_tensor_scale_plan": ([_I64, _I64, _I64, ctypes.POINTER(ctypes.c_int32)], _I),
     "wush_gemm_s4": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _SZ, _P], _I),
@@ -87,6 +89,15 @@ def gemm_s4_workspace_bytes(M, N, K) -> int:
 
 def gemm_s4_best_workspace_bytes(M, N, K) -> int:
     return int(load().wush_gemm_s4_best_workspace_bytes(M, N, K))
+
+
+def gemm_s4_rows_workspace_bytes(xq, xs, wq, ws, M, N, K, rows) -> int:
+    return int(load().wush_gemm_s4_rows_workspace_bytes(xq, xs, wq, ws, M, N, K, rows))
+
+
+def gemm_s4_rows(xq, xs, wq, ws, y, M, N, K, rows, workspace, workspace_bytes, stream) -> None:
+    _check(load().wush_gemm_s4_rows(xq, xs, wq, ws, y, M, N, K, rows, workspace, workspace_bytes, stream),
+           "wush_gemm_s4_rows")
 
 
 # kernels of gemm_s4_plan and gemm_s4_tensor_scale_plan

@@ -134,6 +134,31 @@ bool gemv_preferred(int64_t M, int64_t N, int64_t K) {
     return wush_gemv_int4_supported(M, N, K) != 0 && (M <= 4 || N > 32768);
 }
 
+// The product where the workspace of its plan does not fit the free memory:
+// the same plan over fewer rows at a time, so that the result's bits do not
+// depend on the memory that happens to be free.  Out of memory only if the
+// workspace of 64 rows does not fit either.
+torch::Tensor product_by_rows(const torch::Tensor& xq2, const torch::Tensor& xs2, const torch::Tensor& wq,
+                              const torch::Tensor& ws, torch::Tensor y, int64_t M, int64_t N, int64_t K,
+                              const char* op) {
+    for (int64_t rows = (M + 63) / 64 * 64;; rows = (rows / 2 + 63) / 64 * 64) {
+        const size_t wsb = wush_gemm_s4_rows_workspace_bytes(ptr<uint8_t>(xq2), ptr<uint16_t>(xs2), ptr<uint8_t>(wq),
+                                                             ptr<uint16_t>(ws), M, N, K, rows);
+        torch::Tensor work;
+        try {
+            if (wsb) work = new_tensor({(int64_t)wsb}, torch::kUInt8, xq2);
+        } catch (const c10::OutOfMemoryError&) {
+            if (rows <= 64) throw;
+            continue;
+        }
+        check_status(wush_gemm_s4_rows(ptr<uint8_t>(xq2), ptr<uint16_t>(xs2), ptr<uint8_t>(wq), ptr<uint16_t>(ws),
+                                       ptr<uint16_t>(y), M, N, K, rows, wsb ? work.data_ptr() : nullptr, wsb,
+                                       current_stream(xq2)),
+                     op);
+        return y;
+    }
+}
+
 // Shared product launch: y (M, N) fp16 = group-scaled product, in `sizes`
 // (default (M, N)).
 torch::Tensor product_2d(const torch::Tensor& xq2, const torch::Tensor& xs2, const torch::Tensor& wq,
@@ -148,17 +173,13 @@ torch::Tensor product_2d(const torch::Tensor& xq2, const torch::Tensor& xs2, con
                      op);
         return y;
     }
-    size_t wsb = wush_gemm_s4_best_workspace_bytes(M, N, K);
+    const size_t wsb = wush_gemm_s4_best_workspace_bytes(M, N, K);
     torch::Tensor work;
     if (wsb) {
-        // without room for the fastest plan's workspace, the smaller one's
         try {
             work = new_tensor({(int64_t)wsb}, torch::kUInt8, xq2);
         } catch (const c10::OutOfMemoryError&) {
-            const size_t less = wush_gemm_s4_workspace_bytes(M, N, K);
-            if (less == wsb) throw;
-            wsb = less;
-            if (wsb) work = new_tensor({(int64_t)wsb}, torch::kUInt8, xq2);
+            return product_by_rows(xq2, xs2, wq, ws, y, M, N, K, op);
         }
     }
     check_status(wush_gemm_s4(ptr<uint8_t>(xq2), ptr<uint16_t>(xs2), ptr<uint8_t>(wq), ptr<uint16_t>(ws),

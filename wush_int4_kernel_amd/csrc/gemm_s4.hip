@@ -1062,20 +1062,17 @@ static int plan_kernel(const Plan& p) {
     return p.cfg == 6 ? WUSH_GEMM_FP16_STREAM : p.cfg == 4 ? WUSH_GEMM_INT8_STREAM : WUSH_GEMM_INT8_TILES;
 }
 
+// Whether both scale and both code tensors are 16-byte aligned.
+static bool all_aligned16(const void* xq, const void* xs, const void* wq, const void* ws) {
+    return ((reinterpret_cast<uintptr_t>(xs) | reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(xq) |
+             reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
+}
+
+// Plan p for M rows on a workspace of plan_bytes(p, M, N, K).
 template <bool PT>
-static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
-                    uint16_t* y, int64_t M, int64_t N, int64_t K, void* workspace, size_t ws_bytes,
-                    float alpha, const float* alpha_dev, hipStream_t stream, bool allow_a16 = true) {
-    const bool scales16 = ((reinterpret_cast<uintptr_t>(xs) | reinterpret_cast<uintptr_t>(ws) |
-                            reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
-    // the pre-converted activations need a 16-byte aligned workspace
-    allow_a16 = allow_a16 && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
-    if constexpr (PT) {
-        int rows = 0, cols = 0;
-        if (plan_pt(M, N, K, &rows, &cols))
-            return launch_gemm_pt(xq, wq, y, (int)M, (int)N, (int)K, alpha, alpha_dev, rows, cols, stream);
-    }
-    const Plan p = choose_plan<PT>(M, N, K, workspace ? ws_bytes : 0, scales16, allow_a16);
+static int run_plan(const Plan& p, const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
+                    uint16_t* y, int64_t M, int64_t N, int64_t K, void* workspace, float alpha,
+                    const float* alpha_dev, hipStream_t stream) {
     WUSH_REQUIRE((N + p.tn - 1) / p.tn <= 0x7fffffffLL && (M + p.tm - 1) / p.tm <= 65535);
     float* partial = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     const int m = (int)M, n = (int)N, k = (int)K;
@@ -1123,6 +1120,26 @@ static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, co
         launch_splitk_reduce(partial, y, M * N, p.splits, stream);
     }
     return (int)hipGetLastError();
+}
+
+template <bool PT>
+static int run_gemm(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
+                    uint16_t* y, int64_t M, int64_t N, int64_t K, void* workspace, size_t ws_bytes,
+                    float alpha, const float* alpha_dev, hipStream_t stream, bool allow_a16 = true) {
+    // the pre-converted activations need a 16-byte aligned workspace
+    allow_a16 = allow_a16 && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
+    if constexpr (PT) {
+        int rows = 0, cols = 0;
+        if (plan_pt(M, N, K, &rows, &cols))
+            return launch_gemm_pt(xq, wq, y, (int)M, (int)N, (int)K, alpha, alpha_dev, rows, cols, stream);
+    }
+    const Plan p = choose_plan<PT>(M, N, K, workspace ? ws_bytes : 0, all_aligned16(xq, xs, wq, ws), allow_a16);
+    return run_plan<PT>(p, xq, xs, wq, ws, y, M, N, K, workspace, alpha, alpha_dev, stream);
+}
+
+// The plan of a wush_gemm_s4 call with wush_gemm_s4_best_workspace_bytes.
+static Plan best_plan(int64_t M, int64_t N, int64_t K, bool scales16) {
+    return choose_plan<false>(M, N, K, best_bytes(M, N, K, base_bytes(M, N, K)), scales16, true);
 }
 
 }  // namespace wush
@@ -1177,6 +1194,35 @@ int wush_gemm_s4(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const
                                  stream);
 }
 
+size_t wush_gemm_s4_rows_workspace_bytes(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq,
+                                         const uint16_t* ws, int64_t M, int64_t N, int64_t K, int64_t rows) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 32 || rows <= 0) return 0;
+    const wush::Plan p = wush::best_plan(M, N, K, wush::all_aligned16(xq, xs, wq, ws));
+    return wush::plan_bytes(p, std::min(rows, M), N, K);
+}
+
+int wush_gemm_s4_rows(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
+                      uint16_t* y, int64_t M, int64_t N, int64_t K, int64_t rows, void* workspace,
+                      size_t workspace_bytes, hipStream_t stream) {
+    WUSH_REQUIRE(M >= 0 && N >= 0 && K > 0 && K % 32 == 0);
+    WUSH_REQUIRE(M <= 0x7fffffffLL && N <= 0x7fffffffLL && K <= 0x7fffffffLL);
+    WUSH_REQUIRE(rows > 0 && (rows >= M || rows % 64 == 0));
+    if (M == 0 || N == 0) return (int)hipSuccess;
+    WUSH_REQUIRE(xq && xs && wq && ws && y);
+    WUSH_REQUIRE(((uintptr_t)xq & 15u) == 0 && ((uintptr_t)wq & 15u) == 0);
+    WUSH_REQUIRE(((uintptr_t)xs & 1u) == 0 && ((uintptr_t)ws & 1u) == 0 && ((uintptr_t)y & 1u) == 0);
+    const wush::Plan p = wush::best_plan(M, N, K, wush::all_aligned16(xq, xs, wq, ws));
+    const size_t need = wush::plan_bytes(p, std::min(rows, M), N, K);
+    WUSH_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15u) == 0));
+    // whole 64-row steps keep every operand's and y's alignment
+    for (int64_t r = 0; r < M; r += rows) {
+        const int st = wush::run_plan<false>(p, xq + r * (K / 2), xs + r * (K / 32), wq, ws, y + r * N,
+                                             std::min(rows, M - r), N, K, workspace, 1.0f, nullptr, stream);
+        if (st != 0) return st;
+    }
+    return (int)hipSuccess;
+}
+
 int wush_gemm_s4_noalloc(const uint8_t* xq, const uint16_t* xs, const uint8_t* wq, const uint16_t* ws,
                          uint16_t* y, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
     WUSH_REQUIRE(M >= 0 && N >= 0 && K > 0 && K % 32 == 0);
@@ -1189,8 +1235,7 @@ int wush_gemm_s4_noalloc(const uint8_t* xq, const uint16_t* xs, const uint8_t* w
     // split-K partials only (no pre-converted activations), with fewer K
     // slices where the shape's full split would need more than the scratch
     // (one slice needs none, so every shape has such a plan)
-    const bool scales16 = ((reinterpret_cast<uintptr_t>(xs) | reinterpret_cast<uintptr_t>(ws) |
-                            reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq)) & 15u) == 0;
+    const bool scales16 = wush::all_aligned16(xq, xs, wq, ws);
     const size_t cap = (size_t)WUSH_GEMM_SCRATCH_BYTES;
     const size_t need = wush::plan_bytes(wush::make_plan(M, N, K, cap, true, scales16, false, false), M, N, K);
     if (need > cap) return WUSH_ERROR_SCRATCH_TOO_SMALL;
