@@ -700,19 +700,23 @@ def test_gemm_rows_at_a_time_same_bits(capi, M, N, K):
         capi.gemm_s4_rows(*args, y.data_ptr(), M, N, K, 33 if M > 33 else 0, None, 0, _stream())
 
 
-# Shapes the planner sends to the 256x256 fp16-MFMA tiles (K % 256 == 0,
-# M >= 256, at least 128 tiles): ragged M and N, one and several load batches.
-# The last two split K across workgroups (8 and 4 slices of 8 groups).
-# prefill plans: no K split, and (the last two) ragged M split into 4 and 2
-# slices of 32 groups
-# (200, 40000, 1024): 256-row tiles at 128 < M < 256 (157 column tiles, the
-# last partial).  The last five take the 128-row tiles (N >= 8192, at least
-# 192 workgroups): one row tile of 224 column tiles, K split over 2 slices,
-# a partial column tile (2 slices of 64 groups), 256 column tiles of K=256,
-# and M = 230 (too few 256-row tiles: two 128-row tiles, the second partial).
-H16_SHAPES = [(512, 32768, 256), (700, 30000, 512), (1030, 16400, 1024), (4096, 4096, 2048), (300, 33000, 512),
-              (600, 4096, 4096), (1030, 4096, 2048), (200, 40000, 1024),
-              (65, 57344, 2048), (100, 24576, 4096), (128, 24400, 4096), (128, 65536, 256), (230, 24600, 2048)]
+# Shapes of the fp16-MFMA tiles with a workspace of wush_gemm_s4_workspace_bytes
+# (K % 256 == 0): ragged M and N, one and several load batches; the kernel,
+# tile rows and K slices that the plan query reports for each.
+_CONVERTED, _PER_TILE = 3, 2
+H16_SHAPES = [(512, 32768, 256, (_CONVERTED, 256, 1)), (700, 30000, 512, (_CONVERTED, 128, 1)),
+              (1030, 16400, 1024, (_CONVERTED, 128, 1)), (4096, 4096, 2048, (_PER_TILE, 256, 1)),
+              (300, 33000, 512, (_CONVERTED, 128, 1)), (600, 4096, 4096, (_PER_TILE, 256, 4)),
+              (1030, 4096, 2048, (_PER_TILE, 256, 2)), (200, 40000, 1024, (_CONVERTED, 256, 1)),
+              (65, 57344, 2048, (_CONVERTED, 128, 1)), (100, 24576, 4096, (_CONVERTED, 64, 1)),
+              (128, 24400, 4096, (_CONVERTED, 64, 1)), (128, 65536, 256, (_CONVERTED, 128, 1)),
+              (230, 24600, 2048, (_CONVERTED, 128, 1))]
+
+
+def _plan(capi, M, N, K, wsb=None):
+    """(kernel, tile rows, K slices) with wsb or wush_gemm_s4_workspace_bytes of workspace."""
+    kernel, rows, _, splits = capi.gemm_s4_plan(M, N, K, capi.gemm_s4_workspace_bytes(M, N, K) if wsb is None else wsb)
+    return kernel, rows, splits
 
 
 def _sample(g, n, k):
@@ -739,11 +743,12 @@ def _run_gemm_unaligned(capi, xq, xs, wq, ws):
     return f16_tensor_f64(y)
 
 
-@pytest.mark.parametrize("M,N,K", H16_SHAPES)
-def test_gemm_h16_matches_oracle(capi, M, N, K):
+@pytest.mark.parametrize("M,N,K,plan", H16_SHAPES)
+def test_gemm_h16_matches_oracle(capi, M, N, K, plan):
     # fp16 operands code*scale (exact) with fp32 accumulation over the whole
     # K: seeded samples of rows and columns (first and last always) against
     # the fp64 oracle, for 16-byte and 2-byte aligned scales
+    assert _plan(capi, M, N, K) == plan
     g = rng(4500 + M + N + K)
     xq, xs, wq, ws = _rand_operands(g, M, N, K)
     rows, cols = _sample(g, M, 40), _sample(g, N, 1500)
@@ -768,19 +773,20 @@ def _abs_product(xq, xs, wq, ws):
     return np.einsum("mng,mg,ng->mn", d, sx, sw, optimize=True)
 
 
-@pytest.mark.parametrize("M,N,K,wide", [(2048, 8192, 4096, False), (300, 33000, 512, False),
-                                         (1030, 16400, 1024, False), (512, 8192, 2048, False),
-                                         (512, 8192, 2048, True), (300, 33000, 512, True)])
-def test_gemm_h16_preconverted_activations_agree(capi, M, N, K, wide):
-    # with a workspace of wush_gemm_s4_workspace_bytes, prefill plans with
-    # N >= 8192 convert the activations once into it (h16_prep_a_kernel, then
-    # gemm_h16q); without that room they are converted per tile
-    # (gemm_h16w8): the same fp16 operands, every product exact in fp32,
-    # summed in another order.  So the two outputs differ by at most the two
-    # fp32 sums' rounding (2 * K * 2^-24 * sum |x * w|, generous) plus one
-    # fp16 rounding, on every sampled output.  (512, 8192, 2048) also splits
-    # K (2 slices), compared against the no-alloc entry point, whose scratch
-    # holds the partials but not the converted activations.
+@pytest.mark.parametrize("M,N,K,wide,plan", [
+    (2048, 8192, 4096, False, (256, 1)), (300, 33000, 512, False, (128, 1)), (1030, 16400, 1024, False, (128, 1)),
+    (512, 8192, 2048, False, (64, 1)), (512, 8192, 2048, True, (64, 1)), (300, 33000, 512, True, (128, 1)),
+    (203, 8195, 8192, True, (256, 4)), (131, 8198, 8192, True, (64, 2)), (203, 8195, 8256, True, (256, 4)),
+    (129, 6146, 6144, True, (128, 4))])
+def test_gemm_h16_preconverted_activations_agree(capi, M, N, K, wide, plan):
+    # with a workspace of wush_gemm_s4_best_workspace_bytes, prefill plans
+    # convert the activations once into it (h16_prep_kernel, then
+    # gemm_h16q_kernel); without a workspace they are converted per tile
+    # (gemm_h16w8_kernel: the same fp16 operands) or the int8 tiles run: every
+    # product exact in fp32, summed in another order.  So the two outputs
+    # differ by at most the two fp32 sums' rounding (2 * K * 2^-24 * sum |x * w|,
+    # generous) plus one fp16 rounding, on every sampled output.  Plans with
+    # several K slices have shifts of their own per slice.
     import torch
     # wide: activation scales spanning 2^35 within a row, so that tiny ones
     # reach fp16's subnormal range and the per-slice shift matters
@@ -790,19 +796,16 @@ def test_gemm_h16_preconverted_activations_agree(capi, M, N, K, wide):
     else:
         xq, xs, wq, ws = _rand_operands(g, M, N, K)
     dx, dxs, dw, dws = _dev_operands(xq, xs, wq, ws)
-    wsb = capi.gemm_s4_workspace_bytes(M, N, K)
-    assert wsb >= 2 * M * K, "the plan should hold the converted activations"
+    wsb = capi.gemm_s4_best_workspace_bytes(M, N, K)
+    assert _plan(capi, M, N, K, wsb) == (capi.FP16_CONVERTED, *plan)
+    assert _plan(capi, M, N, K, 0)[0] in (capi.FP16_TILES, capi.INT8_TILES)
     work = torch.empty(wsb, dtype=torch.uint8, device="cuda")
     y_a = torch.empty(M, N, dtype=torch.float16, device="cuda")
     capi.gemm_s4(dx.data_ptr(), dxs.data_ptr(), dw.data_ptr(), dws.data_ptr(), y_a.data_ptr(), M, N, K,
                  work.data_ptr(), wsb, _stream())
     y_t = torch.empty(M, N, dtype=torch.float16, device="cuda")
-    if wsb > 4 * M * K:   # split-K partials too
-        capi.gemm_s4_noalloc(dx.data_ptr(), dxs.data_ptr(), dw.data_ptr(), dws.data_ptr(), y_t.data_ptr(),
-                             M, N, K, _stream())
-    else:
-        capi.gemm_s4(dx.data_ptr(), dxs.data_ptr(), dw.data_ptr(), dws.data_ptr(), y_t.data_ptr(), M, N, K,
-                     None, 0, _stream())
+    capi.gemm_s4(dx.data_ptr(), dxs.data_ptr(), dw.data_ptr(), dws.data_ptr(), y_t.data_ptr(), M, N, K,
+                 None, 0, _stream())
     torch.cuda.synchronize()
     ya, yt = f16_tensor_f64(y_a), f16_tensor_f64(y_t)
     assert np.isfinite(ya).all() and np.isfinite(yt).all()
@@ -819,13 +822,16 @@ def test_gemm_h16_preconverted_activations_agree(capi, M, N, K, wide):
     assert rel_fro(t, ref) < FRO_TOL
 
 
-@pytest.mark.parametrize("M,N", [(512, 32768), (128, 65536)])
-def test_gemm_h16_int_exact_and_group_dots(capi, M, N):
+H16_TILE_SHAPES = [(512, 32768, 256), (128, 65536, 128), (129, 33001, 64)]   # M, N, tile rows at K = 256
+
+
+@pytest.mark.parametrize("M,N,tile", H16_TILE_SHAPES)
+def test_gemm_h16_int_exact_and_group_dots(capi, M, N, tile):
     # unit scales and small codes: integer sums, exact in fp16; then scales 1
-    # on one group only and 0 elsewhere: y = D[:, :, g] exactly (M=128: the
-    # 128-row tiles)
+    # on one group only and 0 elsewhere: y = D[:, :, g] exactly
     g = rng(4510 + M)
     K = 256
+    assert _plan(capi, M, N, K) == (capi.FP16_CONVERTED, tile, 1)
     xq = pack_codes(g.integers(-2, 3, (M, K)))
     wq = pack_codes(g.integers(-2, 3, (N, K)))
     xs = np.full((M, K // 32), 0x3F80, np.uint16)
@@ -874,27 +880,25 @@ def test_gemm_h16_group_dots_nonunit_scales(capi):
         assert np.array_equal(y, exact), gg
 
 
-@pytest.mark.parametrize("M,N", [(512, 32768), (128, 65536)])   # 256-row and 128-row tiles
-def test_gemm_h16_group_scale_boundary(capi, M, N):
+@pytest.mark.parametrize("M,N,tile", H16_TILE_SHAPES)
+def test_gemm_h16_group_scale_boundary(capi, M, N, tile):
     # One activation group at 2^-k of its row's largest scale (full 8-bit
     # significands; the largest sits in group 0, whose codes are 0), one weight
     # group nonzero.  The shifted largest scale lies in [2^12, 2^13), so the
     # fp16 scale operand of the tested group keeps all 8 bits (lowest bit at
-    # or above 2^-24) down to k = 29: y = fp16(sx * sw * D) exactly.  Below,
-    # it rounds to fp16's subnormal spacing: each product term is off by at
-    # most 2^-31 * sx_max * sw_max (2^-27 taken: generous), on top of the fp32
-    # sum of 32 terms and the fp16 rounding of y.
+    # or above 2^-24) down to k = 29; below, its rows' outputs are computed
+    # apart, in fp64.  Either way y = fp16(sx * sw * D) exactly (the product has
+    # at most 8 + 3 + 11 bits).
     g = rng(4516 + M)
     K = 256
     G = K // 32
+    assert _plan(capi, M, N, K) == (capi.FP16_CONVERTED, tile, 1)
     xq, _, wq, _ = _rand_operands(g, M, N, K)
     codes = unpack_codes(xq)
     codes[:, :32] = 0
     xq = pack_codes(codes)
     rows, cols = _sample(g, M, 64), _sample(g, N, 2048)
     D = oracle.group_dots(xq[rows], wq[cols]).astype(np.float64)
-    A = oracle.group_dots(pack_codes(np.abs(unpack_codes(xq[rows]))),
-                          pack_codes(np.abs(unpack_codes(wq[cols])))).astype(np.float64)
     top = (((127 + g.integers(-2, 1, M)) << 7) | g.integers(0, 128, M)).astype(np.uint16)   # [0.25, 2)
     for k in (22, 25, 26, 29, 30, 33):
         gg = 1 + k % (G - 1)
@@ -907,16 +911,9 @@ def test_gemm_h16_group_scale_boundary(capi, M, N):
         sx = bf16_bits_to_f32(xs[rows, gg]).astype(np.float64)
         sw = bf16_bits_to_f32(ws[cols, gg]).astype(np.float64)
         exact = sx[:, None] * sw[None, :] * D[:, :, gg]
-        if k <= 29:
-            assert np.array_equal(y, exact.astype(np.float16).astype(np.float64)), k
-        else:
-            sx_max = bf16_bits_to_f32(top[rows]).astype(np.float64)
-            ulp = np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64)
-            bound = (0.5 * ulp + 32 * 2.0 ** -24 * sx[:, None] * sw[None, :] * A[:, :, gg]
-                     + 32 * 2.0 ** -27 * sx_max[:, None] * sw[None, :])
-            assert (np.abs(y - exact) <= bound).all(), k
-            if (np.abs(exact) >= 2.0 ** -22).any():   # some outputs well inside fp16's range
-                assert np.count_nonzero(y) > 0, k
+        assert np.array_equal(y, exact.astype(np.float16).astype(np.float64)), k
+        if (np.abs(exact) >= 2.0 ** -22).any():   # some outputs well inside fp16's range
+            assert np.count_nonzero(y) > 0, k
 
 
 def _bf16_times_pow2(bits, e):
@@ -926,16 +923,22 @@ def _bf16_times_pow2(bits, e):
     return b.astype(np.uint16)
 
 
-@pytest.mark.parametrize("M,N,K", [(600, 24000, 1024), (100, 49000, 2048)])   # 256-row and 128-row tiles
-def test_gemm_h16_scale_range(capi, M, N, K):
+@pytest.mark.parametrize("M,N,K,plan", [(600, 24000, 1024, (128, 1)), (100, 49000, 2048, (128, 1)),
+                                        (200, 40000, 1024, (256, 1)), (203, 8195, 8192, (256, 4)),
+                                        (130, 8196, 6144, (64, 2)), (130, 16390, 4288, (64, 1)),
+                                        (203, 8195, 8256, (256, 4))])
+def test_gemm_h16_scale_range(capi, M, N, K, plan):
     # Scales far outside fp16's range (activation rows near 2^+40, weight
     # columns near 2^-40, and a spread of 2^-12..2^+12 across the groups of a
     # row) so that every row and column needs its own power-of-two shift; the
     # products stay in fp16 range.  Compared with the oracle after removing
     # each row's and column's factor.
+    assert _plan(capi, M, N, K) == (capi.FP16_CONVERTED, *plan)
     g = rng(4520 + M)
     xq, xs, wq, ws = _rand_operands(g, M, N, K)
-    dr = g.integers(-3, 2, M)                    # outputs |y| < 2^11 * 2^2 stay finite in fp16
+    # outputs |y| < 2^11 * 2^2 stay finite in fp16 at K <= 2048; a sum over more
+    # groups grows at most in proportion, which the rows' factors take back
+    dr = g.integers(-3, 2, M) - max(0, int(np.ceil(np.log2(K / 2048))))
     dc = g.integers(-3, 2, N)
     spread = g.integers(-12, 13, (M, K // 32))
     xs2 = _bf16_times_pow2(xs, 40 + dr[:, None] + spread)
@@ -948,14 +951,15 @@ def test_gemm_h16_scale_range(capi, M, N, K):
     assert rel_fro(got, ref) < FRO_TOL, rel_fro(got, ref)
 
 
-@pytest.mark.parametrize("M,N", [(512, 32768), (120, 57344)])   # 256-row and 128-row tiles
-def test_gemm_h16_nonfinite_scales(capi, M, N):
+@pytest.mark.parametrize("M,N,tile", [(512, 32768, 256), (120, 57344, 128), (512, 8192, 64)])
+def test_gemm_h16_nonfinite_scales(capi, M, N, tile):
     # a non-finite activation scale makes its row NaN, a non-finite weight
     # scale its column, as in the dequantized product; the rest is unaffected
     g = rng(4530 + M)
-    K = 512
+    K = 2048 if tile == 64 else 512
+    assert _plan(capi, M, N, K) == (capi.FP16_CONVERTED, tile, 1)
     xq, xs, wq, ws = _rand_operands(g, M, N, K)
-    bad_r, bad_c = [3, M - 12], [5, 20000]
+    bad_r, bad_c = [3, M - 12], [5, min(20000, N - 3)]
     xs[bad_r[0], 2] = 0x7F80                     # +inf
     xs[bad_r[1], 15] = 0xFFC0                    # NaN
     ws[bad_c[0], 1] = 0x7FC0                     # NaN
