@@ -398,7 +398,7 @@ def main():
         def launch_product(kind, M_, N_, K_, wq_, ws_, reps=3):
             xq_, xs_ = _C.quant_int4(activations_k(M_, K_))
             y_ = torch.empty(M_, N_, dtype=torch.float16, device=dev)
-            wsb = capi.gemm_s4_workspace_bytes(M_, N_, K_)
+            wsb = (capi.gemm_s4_best_workspace_bytes if kind == "best" else capi.gemm_s4_workspace_bytes)(M_, N_, K_)
             work = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
             for _ in range(reps):
                 if kind == "gemv":
@@ -422,8 +422,13 @@ def main():
         Wq8, Ws8 = _C.quant_int4((torch.randn(24576, 4096, generator=gdev, device=dev) * 0.02).to(torch.bfloat16))
         launch_product("gemm", 8, 24576, 4096, Wq8, Ws8)   # Qwen3-8B M=8 (K-split streaming GEMM, 8 rows)
         W3, S3 = _C.quant_int4((torch.randn(4096, 4096, generator=gdev, device=dev) * 0.02).to(torch.bfloat16))
-        launch_product("gemm", 4096, 4096, 4096, W3, S3)  # 4096^3 prefill tiles
-        del W3, S3
+        launch_product("gemm", 4096, 4096, 4096, W3, S3)  # 4096^3, operands converted per tile
+        launch_product("best", 4096, 4096, 4096, W3, S3)  # ... activations converted once, as the _C ops run it
+        Xt = activations_k(512, 4096)                      # the per-tensor route at a prefill chunk
+        inv = torch.tensor([2.0], device=dev)
+        for _ in range(3):
+            _C.w4a4_gemm_cutlass_dev(_C.quant_int4_tensor_scale_dev(Xt, inv), Wq8, inv)
+        del W3, S3, Xt
         # L70 M=4096 prefill and hipBLASLt bf16 at the same shape: the clock
         # (GRBM_GUI_ACTIVE) and MFMA-busy comparison of the two
         launch_product("gemm", 4096, N, K, wq, ws)
@@ -472,7 +477,7 @@ def main():
             "mfma": mfma,
             "mfma_tops": round(tflops, 2),
             "mfma_frac": round(tflops / peak, 4),
-            # the north star's roofline for prefill-sized GEMM: the int8 MFMA peak
+            # a prefill-sized GEMM against the int8 MFMA peak
             "int8_peak_frac": round(tflops / INT8_PEAK_TOPS, 4),
         }
         if blas_w is not None:

@@ -129,10 +129,11 @@ size_t wush_gemm_s4_best_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * after a power-of-two shift per row and column, for scales down to 2^-29 of
  * the row's or column's largest; with converted activations the outputs of
  * rows and columns beyond that are computed apart, in fp64, otherwise such
- * scales lose low bits) accumulated in fp32 over all of K: M > 64 with K % 64 == 0, from about 2^32 multiply-adds (3e9, 4.8e9 for
- * N < 2048; twice that for K % 256 != 0; or 192 tiles of 128 x 256 outputs at
- * N >= 8192 and K % 256 == 0), when the workspace holds the converted activations (see the two functions above); without that
- * room M > 128 with K % 256 == 0, at least 64 tiles of 256x256 or N >= 2048, and
+ * scales lose low bits) accumulated in fp32 over all of K: M > 64 with
+ * K % 64 == 0, from about 2^32 multiply-adds (3e9, 4.8e9 for N < 2048; twice
+ * that for K % 256 != 0; or 192 tiles of 128 x 256 outputs at N >= 8192 and
+ * K % 256 == 0), when the workspace holds the converted activations (see the
+ * two functions above); without that room M > 128 with K % 256 == 0, at least 64 tiles of 256x256 or N >= 2048, and
  * at least 128 workgroups counting the K slices of at least 32 groups each
  * that the workspace holds from M = 512; and 32 < M <= 64 with 49953 <= N <=
  * 57344 and K % 1024 == 0 (16-byte aligned codes and scales).

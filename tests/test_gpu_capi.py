@@ -5,7 +5,7 @@ torch supplies device memory and the stream only.  Bars:
     and the committed fixtures;
   * GEMV / GEMM: the int32 group dots exact (unit scales, |Y| < 2048 so fp16
     holds them exactly) and the fp16 output within 2e-3 relative Frobenius of
-    the fp64 dequantized product (the tolerance the north star states);
+    the fp64 dequantized product (the parity tolerance);
   * MFMA layout self-test exact.
 """
 from __future__ import annotations

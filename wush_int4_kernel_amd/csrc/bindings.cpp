@@ -39,7 +39,8 @@ c10::SmallVector<int64_t, 6> with_last(const torch::Tensor& t, int64_t last) {
 // allocator: every op here writes its outputs whole.  torch::empty goes
 // through the dispatcher, 1.7 us a tensor against 3.3 us for a kernel launch;
 // with it and views of flat outputs an eager M=1 K=N=4096 layer step (two
-// launches) took 11.6 us of host time, without 8.2.
+// launches) took 11.6 us of host time, without 8.2.  empty_cuda is not one of
+// torch's documented interfaces, and dispatch modes do not see what it allocates.
 torch::Tensor new_tensor(c10::IntArrayRef sizes, at::ScalarType dtype, const torch::Tensor& t) {
     return torch::Tensor(at::detail::empty_cuda(sizes, dtype, t.device(), std::nullopt));
 }

@@ -146,10 +146,6 @@ __device__ __forceinline__ void frag_write(uint8_t* frag, int L, uint4 v) {
     *reinterpret_cast<uint4*>(frag + 16 * L) = v;
 }
 
-// One load batch of a thread: 4 groups of its activation row and weight
-// column.  Scales: with VEC, sa[0..1] / sb[0..1] hold the 4 bf16 scales as
-// two packed pairs (one 8-byte load per row); otherwise sa[i] / sb[i] hold
-// group i's bf16 bits.
 // Value of the partner lane's `other` (DPP quad permutation CTRL: 0xB1 =
 // [1,0,3,2], lane ^ 1; 0x4E = [2,3,0,1], lane ^ 2) where take_other, else keep.
 template <int CTRL>
@@ -158,8 +154,10 @@ __device__ __forceinline__ uint32_t h16_xchg(uint32_t keep, uint32_t other, bool
     return take_other ? v : keep;
 }
 
-// fp32 value of scale i of a batch (bits are only re-read here, at the
-// conversion, so the load's wait lands there too)
+// fp32 value of scale i of a load batch (4 groups of a row): with VEC, v[0..1]
+// hold the 4 bf16 scales as two packed pairs (one 8-byte load), otherwise v[i]
+// holds group i's bits.  They are only re-read here, at the conversion, so the
+// load's wait lands there too.
 template <bool VEC>
 __device__ __forceinline__ float h16_batch_scale(const uint32_t (&v)[kH16Batch], int i) {
     if constexpr (VEC) return __uint_as_float((i & 1) ? (v[i >> 1] & 0xffff0000u) : (v[i >> 1] << 16));

@@ -4,16 +4,17 @@
 // in gemm_h16.hip).
 //
 // Workgroup: 4 wavefronts side by side over 256 weight columns, wavefront w
-// owning all of the tile's rows (256 or 128) and columns 64w .. 64w + 63.
+// owning all of the tile's rows (256, 128 or 64) and columns 64w .. 64w + 63.
 // Because no other wavefront needs its columns, a wavefront converts its
 // weight codes straight into MFMA operand registers: no LDS traffic for
 // converted weights.  The activations, converted once by h16_prep_kernel in
 // the matching layout, are DMA'd into a 4-slot LDS ring and read by all four.
 //
-// What bounds it on MI355X: power.  At L70 M=4096 an MFMA-only loop of the
-// same tile runs at 1.5-1.6 PFLOP/s with the clock near 1.5 GHz, so the MFMA
-// form matters: v_mfma_f32_16x16x32_f16 moves a third less accumulator data
-// per flop than the 32x32x16 form and the same loop ran 7-10% faster with it
+// What bounds it on MI355X: power (the clock is 2.0 GHz at 4096 cubed with the
+// MFMA pipes 62% busy, 1.6-1.7 at L70 M=4096 with 76%).  There an MFMA-only
+// loop of the same tile runs at 1.5-1.6 PFLOP/s with the clock near 1.5 GHz,
+// so the MFMA form matters: v_mfma_f32_16x16x32_f16 moves a third less
+// accumulator data per flop than 32x32x16 and the same loop ran 7-10% faster
 // (4096 x 16384 x 8192, operands in LDS: 907 -> 806 us).  The accumulators
 // are written in place by an asm MFMA: left to the compiler, tiles that do
 // not fill the AGPRs rotate them (each MFMA writing the next one's input),
@@ -35,9 +36,10 @@
 // path about as much as one reading them whole), one DMA per stage.  Every
 // global load of the loop is an LDS DMA issued by asm that the compiler does
 // not see; the kernel counts them itself.  Every stage issues NA activation
-// DMAs and one code DMA, and stage 4 of each 8 one scale DMA more; at a
-// stage's end all but those of the last two stages have landed, so what a
-// stage issues is read three stages later at the earliest.
+// DMAs and one code DMA, and stage 4 of each 8 the scale DMAs (one, or four for
+// a K that is not a multiple of 256); at a stage's end all but those of the
+// last two stages have landed, so what a stage issues is read three stages
+// later at the earliest.
 //
 // Outputs: fp16 through LDS (the ring and code buffers are free after the
 // last stage) as 8-byte writes -- the weights are the MFMA's row operand, so
@@ -100,8 +102,8 @@ __device__ __forceinline__ float h16_exact_output(const uint8_t* __restrict__ xq
     return (float)acc;
 }
 
-// RB: 16-row blocks per wavefront, 16 (256-row tiles) or 8 (128-row tiles:
-// half the accumulators, the same weight conversion per stage) or 4.  PAD: K is
+// RB: 16-row blocks per wavefront, 16 (256-row tiles), 8 or 4 (128- and 64-row
+// tiles: fewer accumulators, the same weight conversion per stage).  PAD: K is
 // a multiple of 64 but not of 256: the last double batch reads the row's last
 // groups again in place of those past the end, whose activations and weight
 // scales are zero, and scales come 4 bytes at a time (rows of them are only

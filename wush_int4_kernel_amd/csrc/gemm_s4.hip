@@ -842,10 +842,10 @@ static bool h16a_preferred(int64_t M, int64_t N, int64_t K) {
 // per CU) a fixed cost (ring fill, epilogue) and a cost per 32-wide stage that
 // grows with the workgroups running (`lo` alone, `hi` with the chip full: the
 // clock follows the power), the conversion's bytes at 5 TB/s, and for s > 1
-// the partials' write, read and launch.  Fitted to 64 shapes (64 <= M <= 4096,
-// 512 <= N <= 65536, 256 <= K <= 16384, every tile height and K split): the
-// tile and split with the least estimate is on average 0.7% slower than the
-// best one measured, 10% at worst.
+// the partials' write, read and launch.  On 64 shapes drawn after the constants
+// were set (65 <= M <= 4096, 512 <= N <= 65536, 256 <= K <= 16384, every tile
+// height and K split timed) the tile and split with the least estimate was the
+// fastest for 54, 1.0% slower than the fastest on average and 11% at worst.
 static double h16a_cost_us(int64_t M, int64_t N, int64_t K, int rows, int s, int groups_per_split) {
     static const struct { int rows; double fixed, lo, hi; } kCost[] = {
         {64, 3.5, 0.225, 0.275}, {128, 4.5, 0.3125, 0.40}, {256, 8.0, 0.50, 0.66}};
