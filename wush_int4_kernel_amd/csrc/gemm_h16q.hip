@@ -51,8 +51,8 @@
 //
 // Rows and columns whose scales span more than the operands hold (h16_loses_bits)
 // are found by the conversion kernel, and a tile ends by computing their
-// outputs from the codes and bf16 scales: nothing is paid for inputs without
-// them but one test per row and column.
+// outputs from the codes and bf16 scales: inputs without them pay one test per
+// row and column.
 //
 // Measured (layer with the fused transform, same box, against the 32x32x16
 // form with burst DMAs): K=8192 N=57344 M=4096 3179 -> 2679 us (1.45 PFLOP/s;
@@ -76,30 +76,66 @@ __device__ __forceinline__ bool h16_loses_bits(uint32_t bits, uint32_t mx) {
     return (int)(mx >> 7) - max((int)(bits >> 7), 1) > 29;
 }
 
-// Output (m, n) over groups [g0, g1) from the codes and bf16 scales: exact
-// int32 group dots summed in fp64.  For the outputs of wide rows and columns
-// only: such inputs are rare, so one lane per output, unblocked, will do.
-__device__ __forceinline__ float h16_exact_output(const uint8_t* __restrict__ xq, const uint16_t* __restrict__ xs,
-                                                  const uint8_t* __restrict__ wq, const uint16_t* __restrict__ ws,
-                                                  int m, int n, int GR, int g0, int g1) {
-    const uint4* x = reinterpret_cast<const uint4*>(xq + (size_t)m * GR * 16);
-    const uint4* w = reinterpret_cast<const uint4*>(wq + (size_t)n * GR * 16);
-    const uint16_t* sx = xs + (size_t)m * GR;
-    const uint16_t* sw = ws + (size_t)n * GR;
-    double acc = 0.0;
-#pragma unroll 1
-    for (int g = g0; g < g1; ++g) {
-        const uint4 a = x[g], b = w[g];
-        int d = __builtin_amdgcn_sdot8((int)a.x, (int)b.x, 0, false);
-        d = __builtin_amdgcn_sdot8((int)a.y, (int)b.y, d, false);
-        d = __builtin_amdgcn_sdot8((int)a.z, (int)b.z, d, false);
-        d = __builtin_amdgcn_sdot8((int)a.w, (int)b.w, d, false);
-        const uint32_t ux = sx[g], uw = sw[g];
-        // a non-finite scale makes its row or column NaN whatever the codes
-        if (max(ux & 0x7fffu, uw & 0x7fffu) >= 0x7f80u) return __builtin_nanf("");
-        acc += (double)d * (double)__uint_as_float(ux << 16) * (double)__uint_as_float(uw << 16);
+// Outputs of R rows (or columns) `u` against each lane's column (or row) `l`,
+// all indexes into (rows, GR) groups of codes and scales: exact int32 dots of
+// groups [g0, g1) summed in fp64; NaN where a scale is not finite, whatever the
+// codes.  For the outputs of wide rows and columns only.  Alone (R = 1) bound by
+// the latency of the lane side's loads, 64 rows of one 16-byte group each, so
+// AHEAD groups go out at a time; by their number where many are wide, so they
+// meet R rows of the other side, whose address is the same in every lane.
+// 2048 x 4096 x 4096, product: 72 us without a wide row, 95 with one, 249 with
+// a tenth of them, 1.5 ms with all (one row and 8 groups at a time: 117, 868,
+// 8.1 ms; the per-tile kernel, which loses the bits, 97).
+template <int R, int AHEAD>
+__device__ __forceinline__ void h16_exact_outputs(const uint8_t* __restrict__ uq, const uint16_t* __restrict__ us,
+                                                  const uint8_t* __restrict__ lq, const uint16_t* __restrict__ ls,
+                                                  const int (&u)[R], int l, int GR, int g0, int g1, float (&out)[R]) {
+    const uint4* lc = reinterpret_cast<const uint4*>(lq) + (size_t)l * GR;
+    const uint16_t* lsc = ls + (size_t)l * GR;
+    double acc[R];
+    uint32_t top[R], ltop = 0;                   // largest scale bits, sign cleared
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        acc[k] = 0.0;
+        top[k] = 0;
     }
-    return (float)acc;
+    auto take = [&](auto nc, int g) {            // groups g .. g + n - 1
+        constexpr int n = nc.value;
+        uint4 b[n];
+        uint32_t sl[n];
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            b[i] = lc[g + i];
+            sl[i] = lsc[g + i];
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const uint4* uc = reinterpret_cast<const uint4*>(uq) + (size_t)u[k] * GR + g;
+            const uint16_t* usc = us + (size_t)u[k] * GR + g;
+#pragma unroll
+            for (int i = 0; i < n; ++i) {
+                const uint4 a = uc[i];
+                const uint32_t w = usc[i];
+                int d = __builtin_amdgcn_sdot8((int)a.x, (int)b[i].x, 0, false);
+                d = __builtin_amdgcn_sdot8((int)a.y, (int)b[i].y, d, false);
+                d = __builtin_amdgcn_sdot8((int)a.z, (int)b[i].z, d, false);
+                d = __builtin_amdgcn_sdot8((int)a.w, (int)b[i].w, d, false);
+                top[k] = max(top[k], w & 0x7fffu);
+                acc[k] += (double)d * ((double)__uint_as_float(w << 16) * (double)__uint_as_float(sl[i] << 16));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < n; ++i) ltop = max(ltop, sl[i] & 0x7fffu);
+    };
+    int g = g0;
+#pragma unroll 1
+    for (; g + AHEAD <= g1; g += AHEAD) take(std::integral_constant<int, AHEAD>{}, g);
+#pragma unroll 1
+    for (; g + 8 <= g1; g += 8) take(std::integral_constant<int, 8>{}, g);
+#pragma unroll 1
+    for (; g < g1; g += 2) take(std::integral_constant<int, 2>{}, g);    // K % 64 == 0: whole pairs
+#pragma unroll
+    for (int k = 0; k < R; ++k) out[k] = max(top[k], ltop) >= 0x7f80u ? __builtin_nanf("") : (float)acc[k];
 }
 
 // RB: 16-row blocks per wavefront, 16 (256-row tiles), 8 or 4 (128- and 64-row
@@ -395,23 +431,37 @@ void gemm_h16q_kernel(const uint8_t* __restrict__ a16, const int* __restrict__ e
         else reinterpret_cast<_Float16*>(y)[(size_t)m * N + n] = (_Float16)v;
     };
     const int ecl = sh_e[256 + wave * 64 + ln];     // one column per lane
-    uint64_t bad = __ballot(ecl == kH16NonFinite), wide = __ballot(ecl == kH16Wide);
+    uint64_t bad = __ballot(ecl == kH16NonFinite);
+    const uint64_t wide_cols = __ballot(ecl == kH16Wide);
     const int g1 = min(GR, gb + groups_per_split);
-    bool waited = false;
-    for (; wide != 0; wide &= wide - 1) {
-        if (!waited) WUSH_WAIT_VMCNT(0);
-        waited = true;
-        const int n = wn0 + __builtin_ctzll(wide);
-        for (int m = m0 + ln; m < min(M, m0 + TR); m += 64)
-            put(m, n, h16_exact_output(xq, xs, wq, ws, m, n, GR, gb, g1));
-    }
-    for (int r = 0; r < TR; r += 64) {
-        for (wide = __ballot(sh_e[r + ln] == kH16Wide); wide != 0; wide &= wide - 1) {
-            if (!waited) WUSH_WAIT_VMCNT(0);
-            waited = true;
-            const int m = m0 + r + __builtin_ctzll(wide);
-            const int n = wn0 + ln;
-            if (n < N) put(m, n, h16_exact_output(xq, xs, wq, ws, m, n, GR, gb, g1));
+    for (int it = 0; it < 2 * (TR / 64); ++it) {
+        // wide rows of 64 against the lanes' columns, then (cols) wide columns
+        // against the lanes' 64 rows
+        const bool cols = it >= TR / 64;
+        const int r = (cols ? it - TR / 64 : it) * 64;
+        uint64_t wide = cols ? wide_cols : __ballot(sh_e[r + ln] == kH16Wide);
+        if (wide == 0) continue;
+        WUSH_WAIT_VMCNT(0);
+        const int l = cols ? m0 + r + ln : wn0 + ln, lim = cols ? M : N;
+        while (wide != 0) {
+            const int base = cols ? wn0 : m0 + r;
+            auto run = [&](auto rc, auto ahead) {
+                constexpr int R = rc.value;
+                int u[R];
+                float v[R];
+#pragma unroll
+                for (int k = 0; k < R; ++k) {    // the last one again where fewer are left
+                    u[k] = base + __builtin_ctzll(wide);
+                    if (k == R - 1 || (wide & (wide - 1)) != 0) wide &= wide - 1;
+                }
+                h16_exact_outputs<R, ahead.value>(cols ? wq : xq, cols ? ws : xs, cols ? xq : wq, cols ? xs : ws, u,
+                                                  min(l, lim - 1), GR, gb, g1, v);
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    if (l < lim) put(cols ? l : u[k], cols ? u[k] : l, v[k]);
+            };
+            if ((wide & (wide - 1)) == 0) run(std::integral_constant<int, 1>{}, std::integral_constant<int, 32>{});
+            else run(std::integral_constant<int, 4>{}, std::integral_constant<int, 8>{});
         }
     }
     if (bad != 0) WUSH_WAIT_VMCNT(0);
