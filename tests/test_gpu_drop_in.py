@@ -419,3 +419,10 @@ def test_error_behaviour(C):
         C.w4a4_gemm_s4(xq, xs, xq, xs)
     with pytest.raises(RuntimeError, match="single row"):
         C.w4a4_gemv(xq, xs, xq, xs)
+    # fewer scale rows than code rows are refused before anything is launched
+    xq, xs = torch.zeros(4, 32, dtype=torch.uint8, device="cuda"), torch.zeros(4, 2, dtype=torch.bfloat16, device="cuda")
+    for op in (C.w4a4_gemm, C.w4a4_gemm_v1, C.w4a4_gemm_v2, C.w4a4_gemm_s4):
+        with pytest.raises(RuntimeError, match="K mismatch"):
+            op(xq, xs[:3].contiguous(), xq, xs)
+        with pytest.raises(RuntimeError, match="K mismatch"):
+            op(xq, xs, xq, xs[:3].contiguous())

@@ -165,6 +165,8 @@ torch::Tensor product_by_rows(const torch::Tensor& xq2, const torch::Tensor& xs2
 torch::Tensor product_2d(const torch::Tensor& xq2, const torch::Tensor& xs2, const torch::Tensor& wq,
                          const torch::Tensor& ws, int64_t K, const char* op, c10::IntArrayRef sizes = {}) {
     const int64_t M = xq2.size(0), N = wq.size(0);
+    // the legacy ops' own checks leave the scale tensors' row counts open
+    TORCH_CHECK(xs2.numel() >= M * (K / 32) && ws.numel() >= N * (K / 32), "K mismatch: fewer scales than groups");
     const at::hip::OptionalHIPGuardMasqueradingAsCUDA guard(xq2.device());
     const int64_t mn[2] = {M, N};
     auto y = new_tensor(sizes.empty() ? c10::IntArrayRef(mn, 2) : sizes, torch::kHalf, xq2);
